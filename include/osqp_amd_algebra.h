@@ -206,6 +206,16 @@ void       osqp_amd_admm_update(OSQPFloat alpha, OSQPVectorf* x, OSQPVectorf* de
  * set_w_given tells the next solve whether it was written. */
 OSQPFloat* osqp_amd_linsys_w_target(LinSysSolver* s);
 void       osqp_amd_linsys_set_w_given(LinSysSolver* s, OSQPInt given);
+/* Runs `iters` whole ADMM iterations (compute_rhs, the linear solve, update_x /
+ * update_z / update_y; rho-vector case) in one launch, from the current x, z,
+ * y in place, with delta_x / delta_y of the last one: for small and medium
+ * problems, where separate launches cost more than their work.  Returns the
+ * iterations queued: `iters`, or 0 when this linsys has no such path or the
+ * PCG has no A x to continue from (the caller then iterates as usual). */
+OSQPInt    osqp_amd_linsys_run(LinSysSolver* s, OSQPInt iters, OSQPFloat alpha, OSQPVectorf* x,
+                               OSQPVectorf* delta_x, OSQPVectorf* z, OSQPVectorf* y, OSQPVectorf* delta_y,
+                               const OSQPVectorf* q, const OSQPVectorf* l, const OSQPVectorf* u,
+                               const OSQPVectorf* rho_inv);
 /* Queued reductions (no counterpart in the reference, whose reductions each
  * return to the host): each call queues the same reduction as
  * OSQPVectorf_norm_inf / scaled_norm_inf / dot_prod / dot_prod_signed (same

@@ -20,7 +20,7 @@ BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libosqp_amd.so")
 MARSHAL = os.path.join(HERE, "_marshal.so")
 
-HIP_SOURCES = ["hip/runtime.hip", "hip/vector.hip", "hip/matrix.hip", "hip/panel.hip", "hip/pcg.hip", "serve/batch.hip"]
+HIP_SOURCES = ["hip/runtime.hip", "hip/vector.hip", "hip/matrix.hip", "hip/panel.hip", "hip/runner.hip", "hip/pcg.hip", "serve/batch.hip"]
 C_SOURCES = ["host/auxil.c", "host/osqp_api.c", "host/polish.c", "host/profilers.c"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -50,6 +50,7 @@
 #include "hip_internal.h"
 #include "spmv_rb.h"
 #include "panel.h"
+#include "runner.h"
 #include "../profilers.h"
 
 using namespace osqp_hip;
@@ -845,6 +846,8 @@ struct HipPcg {
   float* ap;
   float* u;
   int z_incr, z_count, z_use;
+  // the whole loop in one launch, for small and medium problems (runner.h)
+  Runner run;
 };
 
 // solves between two exact recomputations of the cached A x64
@@ -1548,6 +1551,7 @@ void pcg_free(LinSysSolver* self) {
   hybrid_free(&s->hA32); hybrid_free(&s->hK32); hybrid_free(&s->hA64); hybrid_free(&s->hK64);
   dev_free(s->ap); dev_free(s->u);
   dev_free(s->partA); dev_free(s->partK);
+  runner_free(&s->run);
   if (s->h_st) (void)hipHostFree(s->h_st);
   if (s->h_flags) (void)hipHostFree(s->h_flags);
   free(s);
@@ -1663,7 +1667,55 @@ OSQPInt osqp_algebra_init_linsys_solver(LinSysSolver** sp, const OSQPMatrix* P, 
   double cg_bytes = 0.0;
   osqp_amd_linsys_bytes(&s->base, &cg_bytes, nullptr);
   s->lookahead = cg_bytes > 64e6 ? 0 : 2;
+  // The runner multiplies by CG-precision copies throughout: with the FP32 CG
+  // only where the defect correction reads FP32 copies anyway.
+  const bool copies = s->bits == 64 || (s->dcK32 && s->dcA32);
+  if (!polishing && rho_vec && copies && runner_build(&s->run, A, P, RunK{s->krp, s->kci, s->kval64}, s->bits)) {
+    pcg_free(&s->base);
+    *sp = nullptr;
+    return OSQP_LINSYS_SOLVER_INIT_ERROR;
+  }
   return 0;
+}
+
+OSQPInt osqp_amd_linsys_run(LinSysSolver* ls, OSQPInt iters, OSQPFloat alpha, OSQPVectorf* x, OSQPVectorf* delta_x,
+                            OSQPVectorf* z, OSQPVectorf* y, OSQPVectorf* delta_y, const OSQPVectorf* q,
+                            const OSQPVectorf* l, const OSQPVectorf* u, const OSQPVectorf* rho_inv) {
+  HipPcg* s = (HipPcg*)ls;
+  if (!s || !s->run.on || iters <= 0 || s->polishing || !s->rho_vec) return 0;
+  if (!s->ax_valid || s->ax_Aver != s->A->version) return 0;  // the first iteration builds A x64
+  if (s->kver_P != s->P->version || s->kver_A != s->A->version || (s->bits == 32 && s->A->fp32_dirty))
+    update_precond(s);
+  RunCall c;
+  c.iters = iters;
+  c.z_count = s->z_count;
+  c.max_iter = s->max_iter;
+  c.reduction_threshold = s->reduction_threshold;
+  c.guard = s->bits == 32 ? 1 : 0;
+  c.alpha = alpha;
+  c.sigma = s->sigma;
+  c.spr = s->scaled_prim_res ? *s->scaled_prim_res : 0.0;
+  c.sdr = s->scaled_dual_res ? *s->scaled_dual_res : 0.0;
+  c.x = x->d;
+  c.dx = delta_x->d;
+  c.z = z->d;
+  c.y = y->d;
+  c.dy = delta_y->d;
+  c.q = q->d;
+  c.l = l->d;
+  c.u = u->d;
+  c.rho = s->rho_vec->d;
+  c.rhoinv = rho_inv->d;
+  c.x64 = s->x64;
+  c.ax64 = s->ax64;
+  c.dinv = s->dinv;
+  PcgState* st = s->st;
+  c.st = RunState{&st->eps_prev, &st->red_factor, &st->zero_iters, &st->iter, &st->solves, &st->active, &st->done,
+                  &st->total_iters};
+  s->z_count = runner_run(&s->run, s->A, s->P, RunK{s->krp, s->kci, s->kval64}, c);
+  s->host_solves += iters;
+  s->w_given = 0;
+  return iters;
 }
 
 // Times the two CG operator kernels (w = rho o A p and Kp = sigma p + P p + A' w)

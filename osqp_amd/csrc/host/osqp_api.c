@@ -394,6 +394,24 @@ static void print_summary(const OSQPSolver* solver) {
   solver->work->summary_printed = 1;
 }
 
+/* ADMM iterations from `iter` on that the loop of osqp_solve runs without
+ * looking at them on the host: up to the next termination check, rho update,
+ * printed line or the last iteration.  0 where it looks at every one: the
+ * first iteration, a time limit, section markers, a rho interval not yet
+ * fixed, scalar rho. */
+static OSQPInt free_iterations(const OSQPSolver* solver, OSQPInt iter) {
+  const OSQPSettings* s = solver->settings;
+  OSQPInt k = s->max_iter - iter + 1, every[3], j;
+  if (iter == 1 || !s->rho_is_vec || s->profiler_level || s->time_limit < OSQP_TIME_LIMIT) return 0;
+  if (s->adaptive_rho != OSQP_ADAPTIVE_RHO_UPDATE_DISABLED && s->adaptive_rho_interval == 0) return 0;
+  every[0] = s->check_termination;
+  every[1] = s->adaptive_rho != OSQP_ADAPTIVE_RHO_UPDATE_DISABLED ? s->adaptive_rho_interval : 0;
+  every[2] = s->verbose ? OSQP_PRINT_INTERVAL : 0;
+  for (j = 0; j < 3; j++)
+    if (every[j] > 0) k = c_min(k, every[j] - (iter - 1) % every[j]);
+  return c_min(k, 64);  /* an interrupt is seen between launches */
+}
+
 /* ---- solve: src/osqp_api.c:636-1038 ---------------------------------------- */
 OSQPInt osqp_solve(OSQPSolver* solver) {
   OSQPInt exitflag = 0, iter, can_check = 0, can_adapt = 0, can_print = 0;
@@ -414,6 +432,16 @@ OSQPInt osqp_solve(OSQPSolver* solver) {
   work->rhs_ready = 0;
 
   for (iter = 1; iter <= settings->max_iter; iter++) {
+    OSQPInt ran = free_iterations(solver, iter);
+    if (ran > 0)
+      ran = osqp_amd_linsys_run(work->linsys_solver, ran, settings->alpha, work->x, work->delta_x, work->z, work->y,
+                                work->delta_y, work->data->q, work->data->l, work->data->u, work->rho_inv_vec);
+    if (ran > 0) {
+      iter += ran - 1;
+      work->tol_valid = 0;
+      work->rhs_ready = 0;
+      goto iterated;
+    }
     osqp_amd_sec_push(OSQP_AMD_SEC_ADMM_ITER);
     swap_vectors(&(work->x), &(work->x_prev));
     swap_vectors(&(work->z), &(work->z_prev));
@@ -436,7 +464,7 @@ OSQPInt osqp_solve(OSQPSolver* solver) {
     }
     osqp_amd_sec_pop(OSQP_AMD_SEC_ADMM_UPDATE);
     osqp_amd_sec_pop(OSQP_AMD_SEC_ADMM_ITER);
-
+  iterated:
     /* src/osqp_api.c:728-737 */
     if (osqp_amd_interrupted()) {
       update_status(solver->info, OSQP_SIGINT);

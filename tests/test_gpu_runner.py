@@ -1,0 +1,131 @@
+"""The ADMM runner (many iterations in one launch, osqp_amd/csrc/hip/runner.h)
+against the separate kernels, which a solver with section markers
+(profiler_level 1) runs.
+
+One workgroup: the runner takes every row and dot product in the separate
+kernels' order, so x, y and the counts are the same bits.  Several workgroups:
+other summation orders.  FP64: 60 fixed iterations, whose linear solves both
+end at the same CG iteration; the iterates then differ by accumulated
+rounding, bounded by 60 solves of <= 20 CG iterations at 2^-53 relative each,
+times 1e3 for the conditioning of the equilibrated K (sigma 1e-6 to rho 1e2):
+1.4e-10 < 1e-9.  FP32: both points meet the eps 1e-4 termination test, checked
+by their FP64 KKT certificates.
+"""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+from osqp_amd import OSQP
+from osqp_amd import problems as pr
+
+pytestmark = pytest.mark.gpu
+
+EPS = dict(eps_abs=1e-4, eps_rel=1e-4)
+
+
+def qp(n, m, row, seed, p_row=3, long_rows=0):
+    """Random QP with about `row` entries a row of A; the first `long_rows` rows full."""
+    rng = np.random.default_rng(seed)
+    M = sp.random(n, n, density=min(1.0, p_row / n), random_state=rng, data_rvs=rng.standard_normal, format="csc")
+    A = sp.random(m, n, density=min(1.0, row / n), random_state=rng, data_rvs=rng.standard_normal, format="lil")
+    for r in range(long_rows):
+        A[r, :] = rng.standard_normal(n)
+    return dict(P=sp.triu(M @ M.T + 1e-2 * sp.eye(n), format="csc"), q=rng.standard_normal(n), A=sp.csc_matrix(A),
+                l=-rng.random(m), u=rng.random(m), q2=rng.standard_normal(n))
+
+
+def both(p, precision, second=None, **st):
+    """(x, y, iter, status) of a solve and of a changed re-solve, by the separate kernels and by the runner."""
+    out = []
+    for level in (1, 0):
+        s = OSQP(precision=precision)
+        assert s.setup(p["P"], p["q"], p["A"], p["l"], p["u"], profiler_level=level, **st) == 0
+        res = []
+        for change in (None, second):
+            if change:
+                s.update(**change)
+            r = s.solve()
+            res.append((r.x, r.y, r.info.iter, r.info.status_val))
+        res.append(s.stats().pcg_iters)
+        s.close()
+        out.append(res)
+    return out
+
+
+# (n, m, entries a row, full rows): lone elements, odd and RB-divisible n, the
+# workgroup's width and one above, rows past a panel task, an empty row
+ONE = [(1, 1, 1, 0), (2, 3, 1, 0), (63, 65, 3, 0), (255, 400, 4, 1), (256, 300, 4, 0), (500, 64, 5, 1), (801, 90, 6, 2),
+       (1023, 700, 5, 0), (1024, 1025, 5, 0), (1025, 600, 6, 0), (2047, 300, 3, 0), (2048, 40, 8, 1)]
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("n,m,row,full", ONE)
+def test_one_workgroup_same_bits(n, m, row, full, precision):
+    p = qp(n, m, row, seed=n + m, p_row=1.5, long_rows=full)
+    new_A = np.random.default_rng(1).standard_normal(p["A"].nnz)
+    a, b = both(p, precision, second=dict(q=p["q2"], Ax=new_A), **EPS)
+    assert a[2] == b[2]
+    for u, v in zip(a[:2], b[:2]):
+        assert u[2:] == v[2:]
+        assert np.array_equal(u[0], v[0]) and np.array_equal(u[1], v[1])
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("N", [10, 33, 50])
+def test_mpc_same_bits(N, precision):
+    p = pr.mpc(N, seed=N)
+    l, u = p["l"].copy(), p["u"].copy()
+    l[:12] = u[:12] = np.random.default_rng(N).uniform(-1, 1, 12)
+    a, b = both(p, precision, second=dict(l=l, u=u), **EPS)
+    assert a[2] == b[2]
+    for s, t in zip(a[:2], b[:2]):
+        assert s[2:] == t[2:] and np.array_equal(s[0], t[0]) and np.array_equal(s[1], t[1])
+
+
+# (n, m, entries a row): 32, 64, 128 and 256 workgroups; 1 to 12 elements a
+# thread; fewer columns than workgroups; more rows than threads a workgroup
+MANY = [(200, 4000, 20), (33, 30000, 5), (700, 9001, 30), (1025, 12000, 40), (2049, 9000, 90), (4097, 30001, 70),
+        (6145, 20000, 30), (8191, 24000, 25)]
+
+
+@pytest.mark.parametrize("n,m,row", MANY)
+def test_many_workgroups_fp64(n, m, row):
+    p = qp(n, m, row, seed=n)
+    a, b = both(p, 64, second=dict(q=p["q2"]), eps_abs=1e-30, eps_rel=1e-30, max_iter=60)
+    for u, v in zip(a[:2], b[:2]):
+        assert u[2:] == v[2:]
+        for k in (0, 1):
+            assert np.linalg.norm(u[k] - v[k]) <= 1e-9 * max(1.0, np.linalg.norm(u[k]))
+
+
+@pytest.mark.parametrize("n,m,row", MANY + [(9001, 30000, 25), (12288, 40000, 20)])
+def test_many_workgroups_fp32(n, m, row):
+    p = qp(n, m, row, seed=n)
+    a, b = both(p, 32, second=dict(l=p["l"] - 0.1, u=p["u"] + 0.1), **EPS)
+    for k, prob in enumerate((p, dict(p, l=p["l"] - 0.1, u=p["u"] + 0.1))):
+        assert a[k][3] == b[k][3]
+        if a[k][3] != 1:  # the separate kernels stop at max_iter: no point to certify
+            continue
+        for x, y, _, _ in (a[k], b[k]):
+            c = pr.kkt_certificate(prob, x, y)
+            assert c["prim"] <= 1e-4 + 1e-4 * c["scale_p"]
+            assert c["dual"] <= 1e-4 + 1e-4 * c["scale_d"]
+
+
+def test_rows_out_of_order_stay_on_the_separate_kernels():
+    """Columns whose rows are not ascending: the several-workgroup layout needs the order, so the solve
+    takes the separate kernels and gives the sorted problem's answer."""
+    p = qp(300, 5000, 12, seed=4)
+    A = p["A"].copy()
+    for j in range(A.shape[1]):
+        s = slice(A.indptr[j], A.indptr[j + 1])
+        A.indices[s], A.data[s] = A.indices[s][::-1].copy(), A.data[s][::-1].copy()
+    A.has_sorted_indices = True  # as a C caller passes it: taken as it is
+    r = {}
+    for name, M in (("sorted", p["A"]), ("reversed", A)):
+        s = OSQP(precision=64)
+        assert s.setup(p["P"], p["q"], M, p["l"], p["u"], **EPS) == 0
+        r[name] = s.solve()
+        s.close()
+    assert r["sorted"].info.status_val == r["reversed"].info.status_val == 1
+    assert np.linalg.norm(r["sorted"].x - r["reversed"].x) <= 1e-3 * np.linalg.norm(r["sorted"].x)
