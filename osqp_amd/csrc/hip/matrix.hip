@@ -52,21 +52,19 @@ __global__ void k_rmult_csr(double* val, const int* ci, const double* R, long lo
   GRID_STRIDE(k, nnz) val[k] *= R[ci[k]];
 }
 
-// P full: entry (r,c) scaled by the factor of the triu entry it copies
-__global__ void k_lmult_sym(double* val, const int* rp, const int* ci, const double* L, int rows) {
-  GRID_STRIDE(r, rows) {
-    for (int k = rp[r]; k < rp[r + 1]; ++k) {
-      int c = ci[k];
-      val[k] *= L[r < c ? r : c];
-    }
-  }
-}
-
-__global__ void k_rmult_sym(double* val, const int* rp, const int* ci, const double* R, int rows) {
-  GRID_STRIDE(r, rows) {
-    for (int k = rp[r]; k < rp[r + 1]; ++k) {
-      int c = ci[k];
-      val[k] *= R[r > c ? r : c];
+// P full: entry (r,c) scaled by the factor of the triu entry it copies, L[min]
+// (HI = 0) or R[max] (HI = 1).  One wavefront per row: with one thread per row
+// the scaling of a 500 x 500 full P took 426 + 274 us, bound by the longest
+// row's chain of dependent read-modify-writes, against 5 + 5 us.
+template <int HI>
+__global__ void k_mult_sym(double* val, const int* rp, const int* ci, const double* L, int rows) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const long long nw = (long long)gridDim.x * blockDim.x / kWave;
+  for (long long w = ((long long)blockIdx.x * blockDim.x + threadIdx.x) / kWave; w < rows; w += nw) {
+    const int r = (int)w, e = rp[r + 1];
+    for (int k = rp[r] + lane; k < e; k += kWave) {
+      const int c = ci[k];
+      val[k] *= L[HI ? (r > c ? r : c) : (r < c ? r : c)];
     }
   }
 }
@@ -498,7 +496,9 @@ void OSQPMatrix_mult_scalar(OSQPMatrix* A, OSQPFloat sc) {
 
 void OSQPMatrix_lmult_diag(OSQPMatrix* A, const OSQPVectorf* L) {
   if (A->is_triu) {
-    hipLaunchKernelGGL(k_lmult_sym, dim3(egrid(A->n)), dim3(kBlock), 0, S(), A->val, A->rp, A->ci, L->d, A->n);
+    if (A->n > 0)
+      hipLaunchKernelGGL(k_mult_sym<0>, dim3(grid_for((long long)A->n * kWave, kBlock, 16384)), dim3(kBlock), 0, S(),
+                         A->val, A->rp, A->ci, L->d, A->n);
   } else {
     if (A->m > 0)
       hipLaunchKernelGGL(k_lmult_csr, dim3(grid_for((long long)A->m * kWave, kBlock, 16384)), dim3(kBlock), 0, S(),
@@ -512,7 +512,9 @@ void OSQPMatrix_lmult_diag(OSQPMatrix* A, const OSQPVectorf* L) {
 
 void OSQPMatrix_rmult_diag(OSQPMatrix* A, const OSQPVectorf* R) {
   if (A->is_triu) {
-    hipLaunchKernelGGL(k_rmult_sym, dim3(egrid(A->n)), dim3(kBlock), 0, S(), A->val, A->rp, A->ci, R->d, A->n);
+    if (A->n > 0)
+      hipLaunchKernelGGL(k_mult_sym<1>, dim3(grid_for((long long)A->n * kWave, kBlock, 16384)), dim3(kBlock), 0, S(),
+                         A->val, A->rp, A->ci, R->d, A->n);
   } else {
     if (A->nnz > 0)
       hipLaunchKernelGGL(k_rmult_csr, dim3(egrid(A->nnz)), dim3(kBlock), 0, S(), A->val, A->ci, R->d, (long long)A->nnz);
