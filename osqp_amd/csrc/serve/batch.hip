@@ -58,9 +58,11 @@ struct BTable {
 
 constexpr int kCounterRing = 1024;
 
-template <typename V, bool SL>
+template <typename V, int MODE>
 __device__ void run_entry(const Team& t, BProb& P, const BEntry& E, int iters, int* done_iters) {
-  Solver<V, SL> sv(t, P);
+  Solver<V, MODE> sv(t, P);
+  if constexpr (MODE == kLanes)
+    if (E.cmd != 1) sv.load_slices();
   if (E.cmd == 1) {
     sv.setup();
   } else if (E.cmd == 2) {
@@ -90,14 +92,16 @@ __device__ void run_entry(const Team& t, BProb& P, const BEntry& E, int iters, i
 // working set in registers (about 250 VGPRs, two waves per SIMD) instead of
 // spilling it at 128 (a 1024-thread bound); on the MPC stream that cut the GPU
 // time of the same work by 28 %.
-// SL: with the FP32 CG's slices (size buckets kSlicedBucket and up)
-template <typename V, bool SL>
+// MODE: kSlices with the FP32 CG's slices (size buckets kSlicedBucket and up),
+// kLanes over the lane rows (lane buckets)
+template <typename V, int MODE>
 __global__ __launch_bounds__(512) void k_epoch(BTable* tab, int* counters, int lds_bytes) {
   __shared__ double red[kMaxRedBlocks];
   __shared__ double red2[kMaxRedBlocks];
   extern __shared__ double dyn_lds[];
   __shared__ BProb P;
   __shared__ int slot, done_iters, decision;
+  __shared__ int2 slices[MODE == kLanes ? 3 * kWave : 1];
   Team t;
   t.tid = threadIdx.x;
   t.T = blockDim.x;
@@ -107,6 +111,7 @@ __global__ __launch_bounds__(512) void k_epoch(BTable* tab, int* counters, int l
   t.red = red;
   t.red2 = red2;
   t.flag = &decision;
+  t.slices = slices;
   t.lds = (char*)dyn_lds;
   t.lds_bytes = lds_bytes;
   const int ep = tab->epoch;
@@ -128,7 +133,7 @@ __global__ __launch_bounds__(512) void k_epoch(BTable* tab, int* counters, int l
     int* dw = (int*)&P;
     for (int i = threadIdx.x; i < (int)(sizeof(BProb) / 4); i += blockDim.x) dw[i] = sw[i];
     __syncthreads();
-    run_entry<V, SL>(t, P, E, iters, &done_iters);
+    run_entry<V, MODE>(t, P, E, iters, &done_iters);
     __syncthreads();
     int* gw = (int*)E.dev;
     for (int i = threadIdx.x; i < (int)(sizeof(BProb) / 4); i += blockDim.x) gw[i] = dw[i];
@@ -288,7 +293,41 @@ struct GroupDims {
   int ng_short = 0;          // groups of the short rows (all groups without slices)
   int nslice = 0;            // slices of kWave medium rows
   long long ell_slots = 0;   // slice entries: kWave x the slice's width, summed
+  int max_len = 0;           // entries of the longest row
+  bool lanes = false;        // lane rows (set for all three matrices of a problem or none)
+  long long lane_slots = 0;  // their slots
 };
+
+// The lane rows of one CSR (BCsr): each row's first-piece length c0 (its
+// entries up to the next multiple of kGroupPer in its group, as write_groups
+// packs it) and each slice's steps; returns the slots.  Rows of 1..kLaneRow
+// entries only: at most three pieces.
+constexpr int kLaneRow = 2 * kGroupPer + 1;
+constexpr int kLaneMaxRows = kWave * kWave;  // a lane holds one slice's pair
+inline int lane_slices(int rows) { return (rows + kWave - 1) / kWave; }
+long long lane_layout(const int* rp, int rows, unsigned char* c0, int* lsl) {
+  int fill = kGroupSlots;
+  long long at = 0;
+  for (int s = 0; s < lane_slices(rows); ++s) {
+    int pieces = 1, wide = 1;
+    for (int r = s * kWave; r < rows && r < (s + 1) * kWave; ++r) {
+      const int len = rp[r + 1] - rp[r];
+      if (fill + len > kGroupSlots) fill = 0;
+      const int room = kGroupPer - fill % kGroupPer, c = len < room ? len : room;
+      fill += len;
+      if (c0) c0[r] = (unsigned char)c;
+      pieces = std::max(pieces, 1 + (len - c + kGroupPer - 1) / kGroupPer);
+      wide = std::max(wide, c);
+    }
+    const int steps = pieces > 1 ? pieces * kGroupPer : wide > 4 ? 8 : wide > 2 ? 4 : wide;
+    if (lsl) {
+      lsl[2 * s] = (int)at;
+      lsl[2 * s + 1] = steps;
+    }
+    at += (long long)kWave * steps;
+  }
+  return at;
+}
 
 // Size bucket of a problem (one hipGraph and stream each): by
 // w = n + m + nnz(A) + nnz(P), 4096 / 16384 / 65536 / 262144 / 2^20 / more.
@@ -307,6 +346,13 @@ inline int size_bucket(long long n, long long m, long long nnzA, long long nnzP)
 // 25 to 34 us, and MPC problems' epochs took 40 % longer in the kernel that
 // holds the slice path at all.
 constexpr int kSlicedBucket = 3;
+// Problems of the buckets below kLaneBuckets whose rows are all short run in
+// buckets of their own (kBuckets + size bucket), on the kernel over lane rows:
+// 512 MPC problems of horizons 10..50 from 56.8 to 38.9 ms (FP32), 24 of them
+// from 21.0 to 13.1 ms (FP64), the same bits.  Rows over kLaneRow entries need
+// the group walk's split over lanes (portfolios: a 500-entry row a lane would
+// be 500 serial steps), larger problems fill a team's lanes as groups.
+constexpr int kLaneBuckets = 3;
 
 // medium rows in slice order: longest first, row order among equals
 void ell_order(const int* rp, int rows, std::vector<int>* order) {
@@ -329,6 +375,7 @@ GroupDims count_groups(const int* rp, int rows, int cols, bool fp32) {
   for (int r = 0; r < rows; ++r) {
     const int len = rp[r + 1] - rp[r];
     if (len >= kEllMin && len <= kLongRow) nmed++;
+    d.max_len = std::max(d.max_len, len);
   }
   d.ell = fp32 && cols < 65536 && nmed >= kEllMinRows;
   int fill = 0;
@@ -406,6 +453,8 @@ struct Layout {
     size_t loff, lci16, lv32;
     // the FP32 CG's slices of the medium rows (offsets 0 when absent)
     size_t eoff, erl, eci16, ev32;
+    // the lane rows (offsets 0 when absent): lsl, lc0 static, the rest dynamic
+    size_t lsl, lc0, lcol, lrv64, lrv32;
   } gP, gA, gT;
   // dynamic
   size_t ctype, D, Dinv, E, Einv, rho, rhoinv, xa, xb, za, zb, y, xt, zt, dx, dy, Ax, Px, Aty, tn, tm, tn2;
@@ -439,7 +488,7 @@ Layout make_layout(const HostData& h, int vbytes) {
   L.Trp = take(4 * (n + 1));
   L.Tci = take(4 * (size_t)h.nnzA);
   L.Tval = take(8 * (size_t)h.nnzA);
-  auto groups = [&](Layout::Groups* o, const GroupDims& g) {
+  auto groups = [&](Layout::Groups* o, const GroupDims& g, int rows) {
     const size_t slots = (size_t)g.ng * kGroupSlots;
     o->longs = take(4 * (size_t)g.nlong);
     o->empty = take(4 * (size_t)g.nempty);
@@ -452,10 +501,14 @@ Layout make_layout(const HostData& h, int vbytes) {
       o->eoff = take(4 * ((size_t)g.nslice + 1));
       o->erl = take(8 * (size_t)g.nslice * kWave);
     }
+    if (g.lanes) {
+      o->lsl = take(8 * (size_t)lane_slices(rows));
+      o->lc0 = take((size_t)rows);
+    }
   };
-  groups(&L.gP, h.gP);
-  groups(&L.gA, h.gA);
-  groups(&L.gT, h.gT);
+  groups(&L.gP, h.gP, h.n);
+  groups(&L.gA, h.gA, h.m);
+  groups(&L.gT, h.gT, h.n);
   L.q = take(8 * n);
   L.l = take(8 * m);
   L.u = take(8 * m);
@@ -471,6 +524,11 @@ Layout make_layout(const HostData& h, int vbytes) {
     if (g.ell) {
       o->eci16 = take(2 * (size_t)g.ell_slots);
       o->ev32 = take(4 * (size_t)g.ell_slots);
+    }
+    if (g.lanes) {
+      o->lcol = take(2 * (size_t)g.lane_slots);
+      o->lrv64 = take(8 * (size_t)g.lane_slots);
+      if (vbytes == 4) o->lrv32 = take(4 * (size_t)g.lane_slots);
     }
   };
   dyn(&L.gP, h.gP);
@@ -557,6 +615,7 @@ void write_groups(const int* rp, int rows, const GroupDims& d, const Layout::Gro
   std::fill(go0, go0 + slots, (unsigned char)0);
   std::fill(gr0, gr0 + slots, -1);
   int* loff = o.compact ? (int*)(img + (o.loff - base)) : nullptr;
+  if (d.lanes) lane_layout(rp, rows, (unsigned char*)(img + (o.lc0 - base)), (int*)(img + (o.lsl - base)));
   int nl = 0, ne = 0, grp = -1, fill = 0, lpos = 0;
   auto pack = [&](int r) {
     const int len = rp[r + 1] - rp[r];
@@ -657,6 +716,16 @@ Layout build_host(HostData* h, int vbytes, const OSQPCscMatrix* P, const OSQPFlo
   h->gP = count_groups(prp.data(), n, n, sliced);
   h->gA = count_groups(arp.data(), m, n, sliced);
   h->gT = count_groups(A->p, n, m, sliced);
+  // lane rows: small problems of short rows, none empty (MPC and the like)
+  bool lanes = size_bucket(n, m, h->nnzA, h->nnzP) < kLaneBuckets && m > 0;
+  for (const GroupDims* g : {&h->gP, &h->gA, &h->gT})
+    lanes = lanes && g->nempty == 0 && g->max_len <= kLaneRow && std::max(n, m) <= kLaneMaxRows;
+  if (lanes) {
+    for (GroupDims* g : {&h->gP, &h->gA, &h->gT}) g->lanes = true;
+    h->gP.lane_slots = lane_layout(prp.data(), n, nullptr, nullptr);
+    h->gA.lane_slots = lane_layout(arp.data(), m, nullptr, nullptr);
+    h->gT.lane_slots = lane_layout(A->p, n, nullptr, nullptr);
+  }
   h->warm_x = x0 != nullptr;
   h->warm_y = y0 != nullptr;
   const Layout L = make_layout(*h, vbytes);
@@ -786,7 +855,11 @@ constexpr int kBuckets = 6;
 constexpr int kEpochIters = 25;
 constexpr int kEpochItersLight = 15;
 
-int bucket_of(const HostData& h) { return size_bucket(h.n, h.m, h.nnzA, h.nnzP); }
+constexpr int kAllBuckets = kBuckets + kLaneBuckets;
+int bucket_of(const HostData& h) {
+  const int b = size_bucket(h.n, h.m, h.nnzA, h.nnzP);
+  return h.gA.lanes ? kBuckets + b : b;
+}
 
 struct Cand {
   int T, tpc;
@@ -802,11 +875,17 @@ constexpr int kNumCands = sizeof(kCands) / sizeof(kCands[0]);
 // such problems cannot keep busy; their epochs' times also move with the
 // other buckets' epochs running beside them, which can rank such a team first.
 constexpr int kSmallBuckets = 2;
-inline int cands_of(int bucket) { return bucket < kSmallBuckets ? 4 : kNumCands; }
+// The lane buckets try the candidates of 256 and 512 threads: one horizon-50
+// problem's iteration takes 90 us with 256 threads and 69 with 512, a horizon-10
+// one's 50 and 48.
+constexpr int kLaneCand0 = 2;
+inline int cands_of(int bucket) {
+  return bucket >= kBuckets ? kNumCands - kLaneCand0 : bucket < kSmallBuckets ? 4 : kNumCands;
+}
 inline int trials_of(int bucket) { return 2 * cands_of(bucket); }
 inline int cand_of_trial(int bucket, int t) {
   const int nc = cands_of(bucket);
-  return t < nc ? t : 2 * nc - 1 - t;
+  return (bucket >= kBuckets ? kLaneCand0 : 0) + (t < nc ? t : 2 * nc - 1 - t);
 }
 
 struct Bucket {
@@ -827,7 +906,7 @@ struct Bucket {
   double rate[kNumCands] = {0};
   int best = 2;   // 256 x 4 until tuned
   int fixT = 0, fixTpc = 0;  // pinned configuration (osqp_batch_set_team)
-  bool sliced = false;       // runs the kernel with slices (bucket >= kSlicedBucket)
+  int mode = kGroups;        // its kernel: kSlices from kSlicedBucket on (FP32), kLanes in the lane buckets
 };
 
 }  // namespace
@@ -838,7 +917,7 @@ struct Engine {
   int max_active = 4096;
   int cus = 256;
   size_t lds_per_cu = 65536;
-  // per kernel (FP32, FP32 with slices, FP64): team size and dynamic LDS
+  // per kernel mode: team size and dynamic LDS
   // bytes of the last lookup, and the kernel's dynamic-LDS limit as set (only
   // ever raised: the graphs of other buckets may launch with the larger size)
   int lds_T[3] = {0, 0, 0};
@@ -864,7 +943,7 @@ struct Engine {
   std::vector<StageCopy> stage_copies;
   int next_id = 1;
   int n_active = 0;
-  Bucket buckets[kBuckets];
+  Bucket buckets[kAllBuckets];
   long long epochs = 0, admm_iters = 0;
   double gpu_s = 0.0;
   bool failed = false;
@@ -938,7 +1017,7 @@ bool admit(Engine* E, HProb* p) {
   P->set = E->set;
   P->st.phase = kPhaseSetup;
   P->st.rho = E->set.rho0;
-  auto csr = [&](BCsr* M, int rows, const GroupDims& g, const Layout::Groups& o, size_t rp, size_t ci,
+  auto csr = [&](BCsr* M, int lslot, int rows, const GroupDims& g, const Layout::Groups& o, size_t rp, size_t ci,
                  size_t val) {
     M->rows = rows;
     M->ng = g.ng;
@@ -962,10 +1041,17 @@ bool admit(Engine* E, HProb* p) {
     M->erl = g.ell ? (int*)(dev + o.erl) : nullptr;
     M->eci16 = g.ell ? (unsigned short*)(dev + o.eci16) : nullptr;
     M->ev32 = g.ell ? (float*)(dev + o.ev32) : nullptr;
+    M->lslot = lslot;
+    M->nls = g.lanes ? lane_slices(rows) : 0;
+    M->lsl = g.lanes ? (int*)(dev + o.lsl) : nullptr;
+    M->lc0 = g.lanes ? (unsigned char*)(dev + o.lc0) : nullptr;
+    M->lcol = g.lanes ? (unsigned short*)(dev + o.lcol) : nullptr;
+    M->lrv64 = g.lanes ? (double*)(dev + o.lrv64) : nullptr;
+    M->lrv32 = g.lanes && E->bits == 32 ? (float*)(dev + o.lrv32) : nullptr;
   };
-  csr(&P->P, h.n, h.gP, L.gP, L.Prp, L.Pci, L.Pval);
-  csr(&P->A, h.m, h.gA, L.gA, L.Arp, L.Aci, L.Aval);
-  csr(&P->At, h.n, h.gT, L.gT, L.Trp, L.Tci, L.Tval);
+  csr(&P->P, 0, h.n, h.gP, L.gP, L.Prp, L.Pci, L.Pval);
+  csr(&P->A, 1, h.m, h.gA, L.gA, L.Arp, L.Aci, L.Aval);
+  csr(&P->At, 2, h.n, h.gT, L.gT, L.Trp, L.Tci, L.Tval);
   P->Pdiag = (int*)(dev + L.Pdiag);
   P->ctype = (int*)(dev + L.ctype);
 #define DPTR(f) P->f = (double*)(dev + L.f)
@@ -1080,15 +1166,17 @@ bool ensure_table(Engine* E, Bucket& B, size_t count) {
 // kTeamLdsBytes and at most what keeps that team count resident.  A problem
 // whose CG vectors fit keeps them there (same arithmetic either way: the
 // bits do not depend on it).  -1 on a HIP error.
-const void* epoch_fn(const Engine* E, bool sliced) {
-  if (E->bits != 32) return (const void*)k_epoch<double, false>;
-  return sliced ? (const void*)k_epoch<float, true> : (const void*)k_epoch<float, false>;
+const void* epoch_fn(const Engine* E, int mode) {
+  if (E->bits != 32) return mode == kLanes ? (const void*)k_epoch<double, kLanes> : (const void*)k_epoch<double, kGroups>;
+  return mode == kLanes    ? (const void*)k_epoch<float, kLanes>
+         : mode == kSlices ? (const void*)k_epoch<float, kSlices>
+                           : (const void*)k_epoch<float, kGroups>;
 }
 
-int team_lds_bytes(Engine* E, int T, bool sliced) {
-  const int w = E->bits == 32 ? (sliced ? 1 : 0) : 2;
+int team_lds_bytes(Engine* E, int T, int mode) {
+  const int w = mode;
   if (E->lds_T[w] == T) return E->lds_B[w];
-  const void* fn = epoch_fn(E, sliced);
+  const void* fn = epoch_fn(E, mode);
   hipFuncAttributes fa;
   int per_cu = 0;
   if (!ok(E, hipFuncGetAttributes(&fa, fn), "hipFuncGetAttributes") ||
@@ -1116,24 +1204,30 @@ int team_lds_bytes(Engine* E, int T, bool sliced) {
   return bytes;
 }
 
+// the bucket's stream, counters and events: the size buckets' with the engine,
+// a lane bucket's with its first epoch
+bool open_bucket(Engine* E, Bucket& B) {
+  if (B.e1) return true;
+  return ok(E, B.stream ? hipSuccess : hipStreamCreateWithFlags(&B.stream, hipStreamNonBlocking), "stream") &&
+         ok(E, B.counters ? hipSuccess : hipMalloc((void**)&B.counters, sizeof(int) * kCounterRing), "hipMalloc counters") &&
+         ok(E, hipMemsetAsync(B.counters, 0, sizeof(int) * kCounterRing, B.stream), "hipMemset counters") &&
+         ok(E, B.e0 ? hipSuccess : hipEventCreate(&B.e0), "event") && ok(E, hipEventCreate(&B.e1), "event");
+}
+
 bool ensure_graph(Engine* E, Bucket& B, int T, int tpc) {
   if (B.exec && B.g_T == T && B.g_tpc == tpc) return true;
   if (B.exec) hipGraphExecDestroy(B.exec);
   if (B.graph) hipGraphDestroy(B.graph);
   B.exec = nullptr;
   B.graph = nullptr;
-  const bool sliced = E->bits == 32 && B.sliced;
-  const int lds = team_lds_bytes(E, T, sliced);
+  const int lds = team_lds_bytes(E, T, B.mode);
   if (lds < 0) return false;
   if (!ok(E, hipStreamBeginCapture(B.stream, hipStreamCaptureModeThreadLocal), "begin capture")) return false;
   const dim3 grid((unsigned)(tpc * E->cus)), block((unsigned)T);
-  if (E->bits != 32)
-    hipLaunchKernelGGL((k_epoch<double, false>), grid, block, (unsigned)lds, B.stream, B.tab, B.counters, lds);
-  else if (sliced)
-    hipLaunchKernelGGL((k_epoch<float, true>), grid, block, (unsigned)lds, B.stream, B.tab, B.counters, lds);
-  else
-    hipLaunchKernelGGL((k_epoch<float, false>), grid, block, (unsigned)lds, B.stream, B.tab, B.counters, lds);
-  if (!ok(E, hipStreamEndCapture(B.stream, &B.graph), "end capture")) return false;
+  int bytes = lds;
+  void* args[] = {&B.tab, &B.counters, &bytes};
+  const hipError_t launched = hipLaunchKernel(epoch_fn(E, B.mode), grid, block, args, (size_t)lds, B.stream);
+  if (!ok(E, hipStreamEndCapture(B.stream, &B.graph), "end capture") || !ok(E, launched, "epoch kernel")) return false;
   if (!ok(E, hipGraphInstantiate(&B.exec, B.graph, nullptr, nullptr, 0), "graph instantiate")) return false;
   B.g_T = T;
   B.g_tpc = tpc;
@@ -1305,13 +1399,10 @@ OSQPInt osqp_batch_create(OSQPBatch** batch, const OSQPSettings* s, OSQPInt prec
     }
     E->images.alloc.reset(E->images.size);
   }
-  for (int k = 0; k < kBuckets && good; ++k) {
+  for (int k = 0; k < kAllBuckets && good; ++k) {
     Bucket& Bk = E->buckets[k];
-    Bk.sliced = k >= kSlicedBucket;
-    good = ok(E, hipStreamCreateWithFlags(&Bk.stream, hipStreamNonBlocking), "stream") &&
-           ok(E, hipMalloc((void**)&Bk.counters, sizeof(int) * kCounterRing), "hipMalloc counters") &&
-           ok(E, hipMemset(Bk.counters, 0, sizeof(int) * kCounterRing), "hipMemset counters") &&
-           ok(E, hipEventCreate(&Bk.e0), "event") && ok(E, hipEventCreate(&Bk.e1), "event");
+    Bk.mode = k >= kBuckets ? kLanes : k >= kSlicedBucket && E->bits == 32 ? kSlices : kGroups;
+    if (k < kBuckets) good = open_bucket(E, Bk);
   }
   if (!good) {
     osqp_batch_destroy(b);
@@ -1582,8 +1673,8 @@ int finish_bucket(Engine* E, int k) {
     B.rate[cand_of_trial(k, B.trial)] += ms > 0 ? its / (double)ms : 0.0;
     B.trial++;
     if (B.trial == trials_of(k)) {
-      int best = 0;
-      for (int c = 1; c < cands_of(k); ++c)
+      int best = cand_of_trial(k, 0);
+      for (int c = best + 1; c < cand_of_trial(k, 0) + cands_of(k); ++c)
         if (B.rate[c] > B.rate[best]) best = c;
       B.best = best;
     }
@@ -1596,9 +1687,9 @@ int finish_bucket(Engine* E, int k) {
 // or -1 on a HIP error.
 int finish_ready(Engine* E) {
   for (;;) {
-    bool any = false, ready[kBuckets] = {};
+    bool any = false, ready[kAllBuckets] = {};
     int n_ready = 0;
-    for (int k = 0; k < kBuckets; ++k) {
+    for (int k = 0; k < kAllBuckets; ++k) {
       Bucket& B = E->buckets[k];
       if (!B.inflight) continue;
       any = true;
@@ -1614,7 +1705,7 @@ int finish_ready(Engine* E) {
     if (!any) return 0;
     if (n_ready) {
       int done = 0;
-      for (int k = 0; k < kBuckets; ++k)
+      for (int k = 0; k < kAllBuckets; ++k)
         if (ready[k]) done += finish_bucket(E, k);
       return done;
     }
@@ -1670,16 +1761,17 @@ OSQPInt osqp_batch_step(OSQPBatch* b, OSQPInt* completed) {
   E->resumed.clear();
   // launch every idle bucket with work (a bucket's table and active list are
   // left alone while its epoch is in flight)
-  for (int k = 0; k < kBuckets; ++k) {
+  for (int k = 0; k < kAllBuckets; ++k) {
     Bucket& B = E->buckets[k];
     if (B.inflight) continue;
     B.active.insert(B.active.end(), B.incoming.begin(), B.incoming.end());
     B.incoming.clear();
     if (B.active.empty()) continue;
-    if (!ensure_table(E, B, B.active.size())) return OSQP_MEM_ALLOC_ERROR;
+    if (!open_bucket(E, B) || !ensure_table(E, B, B.active.size())) return OSQP_MEM_ALLOC_ERROR;
     B.tab->count = (int)B.active.size();
     B.tab->epoch = ++B.epoch;
-    B.tab->iters = (long long)B.active.size() > 2LL * E->cus ? kEpochIters : kEpochItersLight;
+    // (the lane buckets' iterations are short: their epochs end with the checks)
+    B.tab->iters = k >= kBuckets || (long long)B.active.size() > 2LL * E->cus ? kEpochIters : kEpochItersLight;
     for (size_t i = 0; i < B.active.size(); ++i) {
       HProb* p = E->probs[B.active[i]];
       BEntry& en = B.tab->e[i];
@@ -1771,8 +1863,10 @@ OSQPInt osqp_batch_pending(const OSQPBatch* b) {
 
 OSQPInt osqp_batch_tuning(const OSQPBatch* b, OSQPInt bucket, OSQPInt* team, OSQPInt* tpc) {
   if (!b || bucket < 0 || bucket >= kBuckets) return -1;
-  const Bucket& B = b->e.buckets[bucket];
-  if (B.trial < trials_of(bucket)) return -1;
+  // a size bucket and its lane bucket: the one that has run more epochs
+  const bool lane = bucket < kLaneBuckets && b->e.buckets[kBuckets + bucket].epoch > b->e.buckets[bucket].epoch;
+  const Bucket& B = b->e.buckets[lane ? kBuckets + bucket : bucket];
+  if (B.trial < trials_of(lane ? kBuckets + bucket : bucket)) return -1;
   if (team) *team = B.fixT ? B.fixT : kCands[B.best].T;
   if (tpc) *tpc = B.fixT ? B.fixTpc : kCands[B.best].tpc;
   return 0;
@@ -1781,10 +1875,12 @@ OSQPInt osqp_batch_tuning(const OSQPBatch* b, OSQPInt bucket, OSQPInt* team, OSQ
 OSQPInt osqp_batch_set_team(OSQPBatch* b, OSQPInt bucket, OSQPInt team, OSQPInt tpc) {
   if (!b || bucket < 0 || bucket >= kBuckets || tpc < 1 || tpc > 64) return -1;
   if (team != 64 && team != 128 && team != 256 && team != 512) return -1;
-  Bucket& B = b->e.buckets[bucket];
-  B.fixT = (int)team;
-  B.fixTpc = (int)tpc;
-  B.trial = trials_of(bucket);
+  for (int k : {(int)bucket, bucket < kLaneBuckets ? kBuckets + (int)bucket : (int)bucket}) {
+    Bucket& B = b->e.buckets[k];
+    B.fixT = (int)team;
+    B.fixTpc = (int)tpc;
+    B.trial = trials_of(k);
+  }
   return 0;
 }
 
@@ -1799,11 +1895,11 @@ OSQPInt osqp_batch_counters(const OSQPBatch* b, long long* epochs, long long* it
 OSQPInt osqp_batch_destroy(OSQPBatch* b) {
   if (!b) return 0;
   Engine* E = &b->e;
-  for (int k = 0; k < kBuckets; ++k)
+  for (int k = 0; k < kAllBuckets; ++k)
     if (E->buckets[k].stream) hipStreamSynchronize(E->buckets[k].stream);
   for (auto& kv : E->probs) delete kv.second;
   E->probs.clear();
-  for (int k = 0; k < kBuckets; ++k) {
+  for (int k = 0; k < kAllBuckets; ++k) {
     Bucket& B = E->buckets[k];
     if (B.exec) hipGraphExecDestroy(B.exec);
     if (B.graph) hipGraphDestroy(B.graph);

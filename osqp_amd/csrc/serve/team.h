@@ -26,6 +26,8 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "../hip/hip_internal.h"
 
 namespace osqp_serve {
@@ -125,6 +127,21 @@ struct BCsr {
   int* erl;              // nslice * kWave (row, length) pairs
   unsigned short* eci16; // columns (0 for padding)
   float* ev32;           // (float) values, 0 for padding
+  // lane rows (the lane buckets' kernel, which reads no groups): slices of
+  // kWave consecutive rows, one row per lane.  A row's entries are cut where
+  // its group's lanes cut them (multiples of kGroupPer within the group), the
+  // pieces summed in order and added left to right: the additions of the
+  // group walk, so the same bits.  Slice s: lsl[s] = (first slot, steps); step
+  // k of lane l at slot first + kWave k + l; steps 1, 2, 4 or 8 hold one piece
+  // a row, 16 and 24 two and three pieces of kGroupPer.  lc0[r]: entries of
+  // row r's first piece.  Padding: value 0 at the row's first column.
+  int nls;
+  int lslot;             // 0 P, 1 A, 2 A': the matrix's place among the team's LDS slices
+  int* lsl;              // nls (first slot, steps) pairs
+  unsigned char* lc0;    // rows
+  unsigned short* lcol;
+  double* lrv64;
+  float* lrv32;          // (float) values (FP32 engine)
 };
 
 // scalar state that survives between epochs (stored with the problem)
@@ -258,6 +275,7 @@ struct Team {
   double* red;   // LDS, kMaxRedBlocks doubles
   double* red2;  // LDS, kMaxRedBlocks doubles (a second reduction in the same pass)
   int* flag;     // LDS word for decisions that thread 0 takes for the team
+  int2* slices;  // LDS, 3 kWave pairs: the lane rows' slices of P, A, A' (lane buckets)
   __device__ __forceinline__ void sync() const { __syncthreads(); }
   // the team's common value of a decision taken by thread 0 (reads of the
   // device clock differ between threads)
@@ -675,23 +693,103 @@ __device__ __forceinline__ void team_rows(const Team& t, const BCsr M, Elem elem
   }
 }
 
-// y = M x (FP64); caller syncs before reading y
-__device__ __forceinline__ void team_spmv(const Team& t, const BCsr M, const double* __restrict__ x,
-                                          double* __restrict__ y) {
-  team_rows<double>(
-      t, M, [=](double v, int c) { return v * x[c]; }, [=](int r, double s) { y[r] = s; });
+// The same over the lane rows.  What bounds the group walk on rows of a dozen
+// entries is its own row logic (about 46 instructions a slot); here a slot is a
+// value load, a column load, a gather, a product and an addition.
+template <typename TX, typename TV, int K, typename Elem>
+__device__ __forceinline__ TX lane_piece(gptr<const TV> val, gptr<const unsigned short> col, Elem elem) {
+  TV v[K];
+  unsigned short c[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    v[k] = val[k * kWave];
+    c[k] = col[k * kWave];
+  }
+  // every gather issued before the sums
+  TX pr[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) pr[k] = (TX)elem((double)v[k], (int)c[k]);
+  TX tot = 0;
+#pragma unroll
+  for (int g = 0; g < K; g += kGroupPer) {
+    TX acc = pr[g];
+#pragma unroll
+    for (int k = 1; k < (K < kGroupPer ? K : kGroupPer); ++k) acc += pr[g + k];
+    tot = g == 0 ? acc : tot + acc;
+  }
+  return tot;
+}
+// slices: the (first slot, steps) pairs in LDS
+template <typename TX, typename Elem>
+__device__ __forceinline__ TX lane_row(const BCsr& M, const int2* slices, int s, int lane, Elem elem) {
+  using TV = std::conditional_t<sizeof(TX) == 4, float, double>;
+  const int at = __builtin_amdgcn_readfirstlane(slices[s].x) + lane;
+  const int steps = __builtin_amdgcn_readfirstlane(slices[s].y);
+  const gptr<const TV> val = (sizeof(TX) == 4 ? (gptr<const TV>)(const TV*)M.lrv32 : (gptr<const TV>)(const TV*)M.lrv64) + at;
+  const gptr<const unsigned short> col = (gptr<const unsigned short>)M.lcol + at;
+  if (steps == 24) return lane_piece<TX, TV, 24>(val, col, elem);
+  if (steps == 16) return lane_piece<TX, TV, 16>(val, col, elem);
+  if (steps == 8) return lane_piece<TX, TV, 8>(val, col, elem);
+  if (steps == 4) return lane_piece<TX, TV, 4>(val, col, elem);
+  if (steps == 2) return lane_piece<TX, TV, 2>(val, col, elem);
+  return lane_piece<TX, TV, 1>(val, col, elem);
+}
+// epi(row, sum, pre(row)): pre is loaded with the slots, not after the sum
+template <typename TX, typename Elem, typename Pre, typename Epi>
+__device__ __forceinline__ void lane_rows(const Team& t, const BCsr& M, const int2* slices, Elem elem, Pre pre, Epi epi) {
+  for (int s = t.wv; s < M.nls; s += t.W) {
+    const int row = s * kWave + t.lane;
+    const auto w = pre(row < M.rows ? row : 0);
+    const TX r = lane_row<TX>(M, slices, s, t.lane, elem);
+    if (row < M.rows) epi(row, r, w);
+  }
 }
 
 // ---- the ADMM step of one problem -------------------------------------------
 // The problem descriptor is shared by the team (LDS, read-only here); the
 // scalar state S is a private copy in every thread, updated identically by all
 // of them from team-wide reductions (no shared read-modify-write).
-template <typename V, bool SL = false>
+// MODE: how the kernel walks the matrices
+enum : int { kGroups = 0, kSlices = 1, kLanes = 2 };
+
+template <typename V, int MODE = kGroups>
 struct Solver {
   const Team& t;
   const BProb& p;
   BState S;
   __device__ __forceinline__ Solver(const Team& tt, const BProb& pp) : t(tt), p(pp), S(pp.st) {}
+
+  // epi(row, sum of elem over the row) for every row of M; caller syncs
+  template <typename TX, bool CG = false, typename Elem, typename Epi>
+  __device__ __forceinline__ void rows(const BCsr& M, Elem elem, Epi epi) {
+    if constexpr (MODE == kLanes)
+      lane_rows<TX>(
+          t, M, lane_slices(M), elem, [](int) { return 0; }, [=](int r, TX s, int) { epi(r, s); });
+    else
+      team_rows<TX, CG && MODE == kSlices>(t, M, elem, epi);
+  }
+  // the same with a value per row, pre(row)
+  template <typename TX, bool CG = false, typename Elem, typename Pre, typename Epi>
+  __device__ __forceinline__ void rows_with(const BCsr& M, Elem elem, Pre pre, Epi epi) {
+    if constexpr (MODE == kLanes) lane_rows<TX>(t, M, lane_slices(M), elem, pre, epi);
+    else team_rows<TX, CG && MODE == kSlices>(t, M, elem, [=](int r, TX s) { epi(r, s, pre(r)); });
+  }
+  // the slices of P, A and A' in LDS (lane buckets)
+  __device__ __forceinline__ const int2* lane_slices(const BCsr& M) const {
+    return t.slices + M.lslot * kWave;
+  }
+  __device__ __forceinline__ void load_slices() {
+    const BCsr* Ms[3] = {&p.P, &p.A, &p.At};
+    for (int k = 0; k < 3; ++k)
+      for (int i = t.tid; i < Ms[k]->nls; i += t.T)
+        t.slices[Ms[k]->lslot * kWave + i] = ((const int2*)Ms[k]->lsl)[i];
+    t.sync();
+  }
+  // y = M x (FP64); caller syncs before reading y
+  __device__ __forceinline__ void spmv(const BCsr& M, const double* __restrict__ x, double* __restrict__ y) {
+    rows<double>(
+        M, [=](double v, int c) { return v * x[c]; }, [=](int r, double s) { y[r] = s; });
+  }
 
   __device__ __forceinline__ double* x() { return S.swapped ? p.xb : p.xa; }
   __device__ __forceinline__ double* xprev() { return S.swapped ? p.xa : p.xb; }
@@ -866,6 +964,24 @@ struct Solver {
       const unsigned char* __restrict__ goff = M.goff;
       int* __restrict__ gci = M.gci;
       double* __restrict__ gval = M.gval;
+      if constexpr (MODE == kLanes) {
+        // the lane rows' columns and values
+        for (int w = t.tid; w < M.nls * kWave; w += t.T) {
+          const int r = w;
+          const int at = M.lsl[2 * (w / kWave)] + w % kWave, steps = M.lsl[2 * (w / kWave) + 1];
+          const int s0 = r < M.rows ? rp[r] : 0, len = r < M.rows ? rp[r + 1] - s0 : 0, c0 = r < M.rows ? M.lc0[r] : 0;
+          const unsigned short first = len > 0 ? (unsigned short)ci[s0] : (unsigned short)0;
+          for (int k = 0; k < steps; ++k) {
+            const int g = k / kGroupPer, q = g == 0 ? k : c0 + (g - 1) * kGroupPer + k % kGroupPer;
+            const bool in = g == 0 ? k < c0 : q < len;
+            const double v = in ? val[s0 + q] : 0.0;
+            M.lcol[at + k * kWave] = in ? (unsigned short)ci[s0 + q] : first;
+            M.lrv64[at + k * kWave] = v;
+            if (M.lrv32) M.lrv32[at + k * kWave] = (float)v;
+          }
+        }
+        continue;
+      }
       const int slots = M.ng * kGroupSlots;
       for (int i = t.tid; i < slots; i += t.T) {
         const int r = grow[i];
@@ -914,8 +1030,8 @@ struct Solver {
     const double* __restrict__ pval = p.P.val;
     const double sigma = p.set.sigma;
     const int n = p.n;
-    team_rows<double>(
-        t, p.At, [=](double a, int c) { return a * a * rho[c]; }, [=](int r, double s) { prec[r] = s; });
+    rows<double>(
+          p.At, [=](double a, int c) { return a * a * rho[c]; }, [=](int r, double s) { prec[r] = s; });
     t.sync();
     for (int i = t.tid; i < n; i += t.T) {
       const double pd = pdiag[i] >= 0 ? pval[pdiag[i]] : 0.0;
@@ -940,7 +1056,7 @@ struct Solver {
     const gptr<double> w64 = (gptr<double>)p.w64;
     const gptr<double> ax64 = (gptr<double>)p.ax64;
     const gptr<double> gb1 = (gptr<double>)b1, gb2 = (gptr<double>)b2;
-    const BCsr A = p.A, P = p.P, At = p.At;
+    const BCsr &A = p.A, &P = p.P, &At = p.At;
     const bool guard = sizeof(V) == 4;
     // zero-iteration bookkeeping of the previous solve (cuda_pcg_interface.cu:266-268)
     if (S.cg_solves > 0) {
@@ -951,8 +1067,8 @@ struct Solver {
     double eps;
     if (!cached) {
       // rhs64 = b1 + A'(rho o b2); ||rhs64||_inf
-      team_rows<double>(
-          t, At, [=](double v, int c) { return v * (rho[c] * gb2[c]); },
+      rows<double>(
+          At, [=](double v, int c) { return v * (rho[c] * gb2[c]); },
           [=](int row, double s) { rhs64[row] = gb1[row] + s; });
       t.sync();
       const double rhs_norm = norm_inf(p.rhs64, n);
@@ -965,8 +1081,8 @@ struct Solver {
       }
       // w64 = rho o (A x64); r64 = sigma x64 + P x64 + A' w64 - rhs64
       if (m) {
-        team_rows<double>(
-            t, A, [=](double v, int c) { return v * x64[c]; }, [=](int row, double s) { w64[row] = rho[row] * s; });
+        rows<double>(
+          A, [=](double v, int c) { return v * x64[c]; }, [=](int row, double s) { w64[row] = rho[row] * s; });
         t.sync();
       }
       residual64(p.rhs64);
@@ -1003,20 +1119,31 @@ struct Solver {
       if (guard && !(rty > 0.0 && isfinite(rty))) go = false;
       while (go) {
         if (m) {
-          team_rows<V, SL>(
-              t, A, [=](double v, int c) { return (V)v * pp[c]; }, [=](int row, V s) { w[row] = (V)rho[row] * s; });
+          this->template rows_with<V, true>(
+              A, [=](double v, int c) { return (V)v * pp[c]; }, [=](int row) { return (V)rho[row]; },
+              [=](int row, V s, V r) { w[row] = r * s; });
           t.sync();
         }
         // Kp = sigma p + P p + A' w
-        team_rows<V, SL>(
-            t, P, [=](double v, int c) { return (V)v * pp[c]; }, [=](int row, V s) { Kp[row] = s; });
-        t.sync();
-        if (m)
-          team_rows<V, SL>(
-              t, At, [=](double v, int c) { return (V)v * w[c]; },
-              [=](int row, V s) { Kp[row] = (V)sg * pp[row] + Kp[row] + s; });
-        else
-          for (int i = t.tid; i < n; i += t.T) Kp[i] = (V)sg * pp[i] + Kp[i];
+        if constexpr (MODE == kLanes) {
+          // a row of P and the same row of A' by the same lane, in one pass
+          for (int sl = t.wv; sl < P.nls; sl += t.W) {
+            const int row = sl * kWave + t.lane;
+            const V sp = lane_row<V>(P, lane_slices(P), sl, t.lane, [=](double v, int c) { return (V)v * pp[c]; });
+            const V st = lane_row<V>(At, lane_slices(At), sl, t.lane, [=](double v, int c) { return (V)v * w[c]; });
+            if (row < n) Kp[row] = (V)sg * pp[row] + sp + st;
+          }
+        } else {
+          this->template rows<V, true>(
+              P, [=](double v, int c) { return (V)v * pp[c]; }, [=](int row, V s) { Kp[row] = s; });
+          t.sync();
+          if (m)
+            this->template rows<V, true>(
+                At, [=](double v, int c) { return (V)v * w[c]; },
+                [=](int row, V s) { Kp[row] = (V)sg * pp[row] + Kp[row] + s; });
+          else
+            for (int i = t.tid; i < n; i += t.T) Kp[i] = (V)sg * pp[i] + Kp[i];
+        }
         t.sync();
         const double pkp = team_dot<V>(t, n, [=](int i) { return pp[i] * Kp[i]; });
         if (guard && !(pkp > 0.0 && isfinite(pkp))) break;
@@ -1074,8 +1201,8 @@ struct Solver {
     t.sync();
     // b2 = A x64 (the A x cache)
     if (m) {
-      team_rows<double>(
-          t, A, [=](double v, int c) { return v * x64[c]; },
+      rows<double>(
+          A, [=](double v, int c) { return v * x64[c]; },
           [=](int row, double s) {
             ax64[row] = s;
             gb2[row] = s;
@@ -1104,12 +1231,23 @@ struct Solver {
     const double* __restrict__ w64 = p.w64;
     double* __restrict__ tn = p.tn;
     double* __restrict__ r64 = p.r64;
-    team_rows<double>(
-        t, p.P, [=](double v, int c) { return v * x64[c]; }, [=](int row, double s) { tn[row] = s; });
+    if constexpr (MODE == kLanes) {
+      const BCsr &P = p.P, &At = p.At;
+      for (int sl = t.wv; sl < P.nls; sl += t.W) {
+        const int row = sl * kWave + t.lane;
+        const double sp = lane_row<double>(P, lane_slices(P), sl, t.lane, [=](double v, int c) { return v * x64[c]; });
+        const double st = lane_row<double>(At, lane_slices(At), sl, t.lane, [=](double v, int c) { return v * w64[c]; });
+        if (row < n) r64[row] = sigma * x64[row] + sp + st - rhs[row];
+      }
+      t.sync();
+      return;
+    }
+    rows<double>(
+        p.P, [=](double v, int c) { return v * x64[c]; }, [=](int row, double s) { tn[row] = s; });
     t.sync();
     if (p.m)
-      team_rows<double>(
-          t, p.At, [=](double v, int c) { return v * w64[c]; },
+      rows<double>(
+          p.At, [=](double v, int c) { return v * w64[c]; },
           [=](int row, double s) { r64[row] = sigma * x64[row] + tn[row] + s - rhs[row]; });
     else
       for (int i = t.tid; i < n; i += t.T) r64[i] = sigma * x64[i] + tn[i] - rhs[i];
@@ -1149,8 +1287,8 @@ struct Solver {
     if (x0) {
       double* zz = z();
       double* xx = x();
-      team_rows<double>(
-          t, p.A, [=](double v, int c) { return v * xx[c]; }, [=](int row, double s) { zz[row] = s; });
+      rows<double>(
+          p.A, [=](double v, int c) { return v * xx[c]; }, [=](int row, double s) { zz[row] = s; });
       t.sync();
     }
     for (int i = t.tid; i < p.n; i += t.T) p.x64[i] = x()[i];
@@ -1197,7 +1335,7 @@ struct Solver {
   __device__ __forceinline__ double compute_prim_res() {
     double* xx = x();
     const double* zz = z();
-    team_spmv(t, p.A, xx, p.Ax);
+    spmv(p.A, xx, p.Ax);
     t.sync();
     for (int i = t.tid; i < p.m; i += t.T) p.tm[i] = p.Ax[i] - zz[i];
     t.sync();
@@ -1207,8 +1345,8 @@ struct Solver {
   }
   __device__ __forceinline__ double compute_dual_res() {
     double* xx = x();
-    team_spmv(t, p.P, xx, p.Px);
-    if (p.m) team_spmv(t, p.At, p.y, p.Aty);
+    spmv(p.P, xx, p.Px);
+    if (p.m) spmv(p.At, p.y, p.Aty);
     t.sync();
     for (int i = t.tid; i < p.n; i += t.T) {
       double v = p.q[i] + p.Px[i];
@@ -1285,7 +1423,7 @@ struct Solver {
       double lhs = team_reduce<false>(t, p.m, [&](int i) { return p.u[i] * dmax(p.dy[i], 0.0); });
       lhs += team_reduce<false>(t, p.m, [&](int i) { return p.l[i] * dmin(p.dy[i], 0.0); });
       if (lhs < 0.0) {
-        team_spmv(t, p.At, p.dy, p.tn);
+        spmv(p.At, p.dy, p.tn);
         t.sync();
         double nat;
         if (unscaled_term()) nat = team_reduce<true>(t, p.n, [&](int i) { return fabs(p.tn[i] * p.Dinv[i]); });
@@ -1306,13 +1444,13 @@ struct Solver {
     }
     if (ndx > kDivisionTol) {
       if (dot(p.q, p.dx, p.n) < 0.0) {
-        team_spmv(t, p.P, p.dx, p.tn);
+        spmv(p.P, p.dx, p.tn);
         t.sync();
         double npd;
         if (unscaled_term()) npd = team_reduce<true>(t, p.n, [&](int i) { return fabs(p.tn[i] * p.Dinv[i]); });
         else npd = norm_inf(p.tn, p.n);
         if (npd < cs * eps_dinf * ndx) {
-          team_spmv(t, p.A, p.dx, p.tm);
+          spmv(p.A, p.dx, p.tm);
           t.sync();
           if (unscaled_term())
             for (int i = t.tid; i < p.m; i += t.T) p.tm[i] = p.tm[i] * p.Einv[i];
@@ -1406,6 +1544,7 @@ struct Solver {
     for (long long i = t.tid; i < n4; i += t.T) d4[i] = s4[i];
     for (int i = t.tid; i < p.m; i += t.T) p.ctype[i] = 0;
     t.sync();
+    if constexpr (MODE == kLanes) load_slices();
     S.rho = p.set.rho0;
     if (p.set.scaling) scale_data();
     else no_scaling();
