@@ -102,6 +102,7 @@ __global__ __launch_bounds__(512) void k_epoch(BTable* tab, int* counters, int l
   __shared__ BProb P;
   __shared__ int slot, done_iters, decision;
   __shared__ int2 slices[MODE == kLanes ? 3 * kWave : 1];
+  __shared__ int4 longs[MODE == kLanes ? kWave : 1];
   Team t;
   t.tid = threadIdx.x;
   t.T = blockDim.x;
@@ -112,6 +113,7 @@ __global__ __launch_bounds__(512) void k_epoch(BTable* tab, int* counters, int l
   t.red2 = red2;
   t.flag = &decision;
   t.slices = slices;
+  t.longs = longs;
   t.lds = (char*)dyn_lds;
   t.lds_bytes = lds_bytes;
   const int ep = tab->epoch;
@@ -293,7 +295,7 @@ struct GroupDims {
   int ng_short = 0;          // groups of the short rows (all groups without slices)
   int nslice = 0;            // slices of kWave medium rows
   long long ell_slots = 0;   // slice entries: kWave x the slice's width, summed
-  int max_len = 0;           // entries of the longest row
+  int max_len = 0;           // entries of the longest row of at most kLongRow
   bool lanes = false;        // lane rows (set for all three matrices of a problem or none)
   long long lane_slots = 0;  // their slots
 };
@@ -303,6 +305,7 @@ struct GroupDims {
 // packs it) and each slice's steps; returns the slots.  Rows of 1..kLaneRow
 // entries only: at most three pieces.
 constexpr int kLaneRow = 2 * kGroupPer + 1;
+constexpr int kLaneLongs = kWave;  // of A
 constexpr int kLaneMaxRows = kWave * kWave;  // a lane holds one slice's pair
 inline int lane_slices(int rows) { return (rows + kWave - 1) / kWave; }
 long long lane_layout(const int* rp, int rows, unsigned char* c0, int* lsl) {
@@ -312,6 +315,10 @@ long long lane_layout(const int* rp, int rows, unsigned char* c0, int* lsl) {
     int pieces = 1, wide = 1;
     for (int r = s * kWave; r < rows && r < (s + 1) * kWave; ++r) {
       const int len = rp[r + 1] - rp[r];
+      if (len > kLongRow) {  // a wavefront's
+        if (c0) c0[r] = 0;
+        continue;
+      }
       if (fill + len > kGroupSlots) fill = 0;
       const int room = kGroupPer - fill % kGroupPer, c = len < room ? len : room;
       fill += len;
@@ -346,12 +353,13 @@ inline int size_bucket(long long n, long long m, long long nnzA, long long nnzP)
 // 25 to 34 us, and MPC problems' epochs took 40 % longer in the kernel that
 // holds the slice path at all.
 constexpr int kSlicedBucket = 3;
-// Problems of the buckets below kLaneBuckets whose rows are all short run in
+// Problems of the buckets below kLaneBuckets whose rows of P and A' have at
+// most kLaneRow entries, and those of A too or more than kLongRow, run in
 // buckets of their own (kBuckets + size bucket), on the kernel over lane rows:
-// 512 MPC problems of horizons 10..50 from 56.8 to 38.9 ms (FP32), 24 of them
-// from 21.0 to 13.1 ms (FP64), the same bits.  Rows over kLaneRow entries need
-// the group walk's split over lanes (portfolios: a 500-entry row a lane would
-// be 500 serial steps), larger problems fill a team's lanes as groups.
+// 512 MPC problems of horizons 10..50 from 60.0 to 31.9 ms (FP32), 24 of them
+// from 18.6 to 10.7 ms (FP64), 12 resident portfolios of 500..1000 assets from
+// 621 to 300 ms, the same bits.  A row in between has more pieces than the
+// left-to-right sum keeps in the group walk's order.
 constexpr int kLaneBuckets = 3;
 
 // medium rows in slice order: longest first, row order among equals
@@ -375,7 +383,7 @@ GroupDims count_groups(const int* rp, int rows, int cols, bool fp32) {
   for (int r = 0; r < rows; ++r) {
     const int len = rp[r + 1] - rp[r];
     if (len >= kEllMin && len <= kLongRow) nmed++;
-    d.max_len = std::max(d.max_len, len);
+    if (len <= kLongRow) d.max_len = std::max(d.max_len, len);
   }
   d.ell = fp32 && cols < 65536 && nmed >= kEllMinRows;
   int fill = 0;
@@ -719,7 +727,8 @@ Layout build_host(HostData* h, int vbytes, const OSQPCscMatrix* P, const OSQPFlo
   // lane rows: small problems of short rows, none empty (MPC and the like)
   bool lanes = size_bucket(n, m, h->nnzA, h->nnzP) < kLaneBuckets && m > 0;
   for (const GroupDims* g : {&h->gP, &h->gA, &h->gT})
-    lanes = lanes && g->nempty == 0 && g->max_len <= kLaneRow && std::max(n, m) <= kLaneMaxRows;
+    lanes = lanes && g->nempty == 0 && g->max_len <= kLaneRow && g->nlong <= (g == &h->gA ? kLaneLongs : 0) &&
+            std::max(n, m) <= kLaneMaxRows;
   if (lanes) {
     for (GroupDims* g : {&h->gP, &h->gA, &h->gT}) g->lanes = true;
     h->gP.lane_slots = lane_layout(prp.data(), n, nullptr, nullptr);
@@ -876,8 +885,8 @@ constexpr int kNumCands = sizeof(kCands) / sizeof(kCands[0]);
 // other buckets' epochs running beside them, which can rank such a team first.
 constexpr int kSmallBuckets = 2;
 // The lane buckets try the candidates of 256 and 512 threads: one horizon-50
-// problem's iteration takes 90 us with 256 threads and 69 with 512, a horizon-10
-// one's 50 and 48.
+// problem's iteration takes 78 us with 256 threads and 58 with 512, a horizon-10
+// one's 34 and 32; a 1000-asset portfolio's 215 and 166, with 64 threads 657.
 constexpr int kLaneCand0 = 2;
 inline int cands_of(int bucket) {
   return bucket >= kBuckets ? kNumCands - kLaneCand0 : bucket < kSmallBuckets ? 4 : kNumCands;

@@ -232,6 +232,9 @@ using gptr = __attribute__((address_space(1))) T*;
 template <typename T>
 using lptr = __attribute__((address_space(3))) T*;
 
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+
 // ---- DPP lane moves (GFX9 data-parallel primitives) --------------------------
 // v_mov_b32_dpp: each lane reads a register of another lane of its wavefront
 // in the same instruction, without an LDS round trip.  Lanes without a source
@@ -276,6 +279,7 @@ struct Team {
   double* red2;  // LDS, kMaxRedBlocks doubles (a second reduction in the same pass)
   int* flag;     // LDS word for decisions that thread 0 takes for the team
   int2* slices;  // LDS, 3 kWave pairs: the lane rows' slices of P, A, A' (lane buckets)
+  int4* longs;   // LDS, kWave: A's long rows as (row, compact start, CSR start, entries) (lane buckets)
   __device__ __forceinline__ void sync() const { __syncthreads(); }
   // the team's common value of a decision taken by thread 0 (reads of the
   // device clock differ between threads)
@@ -474,8 +478,6 @@ __device__ __forceinline__ void team_rows(const Team& t, const BCsr M, Elem elem
   static_assert(kGroupPer == 8, "a lane's slots are loaded as two int4 / four double2 vectors");
   typedef int i32x4 __attribute__((ext_vector_type(4)));
   typedef double f64x2 __attribute__((ext_vector_type(2)));
-  typedef float f32x4 __attribute__((ext_vector_type(4)));
-  typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
   bool compact = false, sliced = false;
   if constexpr (sizeof(TX) == 4) {
     compact = M.loff != nullptr;
@@ -705,16 +707,17 @@ __device__ __forceinline__ TX lane_piece(gptr<const TV> val, gptr<const unsigned
     v[k] = val[k * kWave];
     c[k] = col[k * kWave];
   }
-  // every gather issued before the sums
-  TX pr[K];
-#pragma unroll
-  for (int k = 0; k < K; ++k) pr[k] = (TX)elem((double)v[k], (int)c[k]);
+  constexpr int kPiece = K < kGroupPer ? K : kGroupPer;
   TX tot = 0;
 #pragma unroll
   for (int g = 0; g < K; g += kGroupPer) {
-    TX acc = pr[g];
+    // a piece's gathers issued before its sum
+    TX pr[kPiece];
 #pragma unroll
-    for (int k = 1; k < (K < kGroupPer ? K : kGroupPer); ++k) acc += pr[g + k];
+    for (int k = 0; k < kPiece; ++k) pr[k] = (TX)elem((double)v[g + k], (int)c[g + k]);
+    TX acc = pr[0];
+#pragma unroll
+    for (int k = 1; k < kPiece; ++k) acc += pr[k];
     tot = g == 0 ? acc : tot + acc;
   }
   return tot;
@@ -734,14 +737,86 @@ __device__ __forceinline__ TX lane_row(const BCsr& M, const int2* slices, int s,
   if (steps == 2) return lane_piece<TX, TV, 2>(val, col, elem);
   return lane_piece<TX, TV, 1>(val, col, elem);
 }
-// epi(row, sum, pre(row)): pre is loaded with the slots, not after the sum
+// A's long rows (LDS list), a wavefront each: the additions of team_rows'
+template <typename TX, typename Elem, typename Pre, typename Epi>
+__device__ __forceinline__ void lane_longs(const Team& t, const BCsr& M, Elem elem, Pre pre, Epi epi) {
+  for (int j = t.W - 1 - t.wv; j < M.nlong; j += t.W) {
+    const int4 L = t.longs[j];
+    const int row = __builtin_amdgcn_readfirstlane(L.x), len = __builtin_amdgcn_readfirstlane(L.w);
+    const auto w = pre(row);
+    TX acc = 0;
+    if constexpr (sizeof(TX) == 4) {
+      const gptr<const float> lv = (gptr<const float>)M.lv32 + __builtin_amdgcn_readfirstlane(L.y);
+      const gptr<const unsigned short> lc = (gptr<const unsigned short>)M.lci16 + __builtin_amdgcn_readfirstlane(L.y);
+      constexpr int kR = 4, kChunk = kWave * kLongVec;
+      for (int k0 = 0; k0 < len; k0 += kR * kChunk) {
+        f32x4 v[kR];
+        u32x2 c[kR];
+#pragma unroll
+        for (int i = 0; i < kR; ++i) {
+          const int k = k0 + i * kChunk + t.lane * kLongVec, kk = k < len ? k : 0;
+          v[i] = *(gptr<const f32x4>)(lv + kk);
+          c[i] = *(gptr<const u32x2>)(lc + kk);
+        }
+#pragma unroll
+        for (int i = 0; i < kR; ++i) {
+          const int k = k0 + i * kChunk + t.lane * kLongVec;
+#pragma unroll
+          for (int q = 0; q < kLongVec; ++q) {
+            const unsigned cc = c[i][q >> 1];
+            const TX pr = (TX)elem((double)v[i][q], (int)((q & 1) ? (cc >> 16) : (cc & 0xFFFFu)));
+            if (k + q < len) acc += pr;
+          }
+        }
+      }
+    } else {
+      const gptr<const double> val = (gptr<const double>)M.val + __builtin_amdgcn_readfirstlane(L.z);
+      const gptr<const int> ci = (gptr<const int>)M.ci + __builtin_amdgcn_readfirstlane(L.z);
+      for (int k0 = t.lane; k0 < len; k0 += kLongPer * kWave) {
+        double v[kLongPer];
+        int c[kLongPer];
+#pragma unroll
+        for (int i = 0; i < kLongPer; ++i) {
+          const int k = k0 + i * kWave < len ? k0 + i * kWave : 0;
+          v[i] = val[k];
+          c[i] = ci[k];
+        }
+#pragma unroll
+        for (int i = 0; i < kLongPer; ++i) {
+          const TX pr = (TX)elem(v[i], c[i]);
+          if (k0 + i * kWave < len) acc += pr;
+        }
+      }
+    }
+    acc = osqp_hip::wave_sum(acc);
+    if (t.lane == 0) epi(row, acc, w);
+  }
+}
+// epi(row, sum, pre(row)): pre is loaded with the slots, not after the sum.
+// A long row's first piece (lc0) is empty: its lane adds padding and writes nothing.
 template <typename TX, typename Elem, typename Pre, typename Epi>
 __device__ __forceinline__ void lane_rows(const Team& t, const BCsr& M, const int2* slices, Elem elem, Pre pre, Epi epi) {
+  const gptr<const unsigned char> lc0 = (gptr<const unsigned char>)M.lc0;
   for (int s = t.wv; s < M.nls; s += t.W) {
-    const int row = s * kWave + t.lane;
-    const auto w = pre(row < M.rows ? row : 0);
+    const int row = s * kWave + t.lane, rr = row < M.rows ? row : 0;
+    const auto w = pre(rr);
+    const bool mine = row < M.rows && (M.nlong == 0 || lc0[rr] != 0);
     const TX r = lane_row<TX>(M, slices, s, t.lane, elem);
-    if (row < M.rows) epi(row, r, w);
+    if (mine) epi(row, r, w);
+  }
+  if (M.nlong) lane_longs<TX>(t, M, elem, pre, epi);
+}
+// use(i, load(i)) for i < n, thread t.tid + k T: kEachU loads in flight
+constexpr int kEachU = 4;
+template <typename Load, typename Use>
+__device__ __forceinline__ void team_each(const Team& t, int n, Load load, Use use) {
+  for (int b = t.tid; b < n; b += kEachU * t.T) {
+    decltype(load(0)) v[kEachU];
+#pragma unroll
+    for (int u = 0; u < kEachU; ++u) v[u] = load(b + u * t.T < n ? b + u * t.T : b);
+#pragma unroll
+    for (int u = 0; u < kEachU; ++u)
+      if (b + u * t.T < n) use(b + u * t.T, v[u]);
   }
 }
 
@@ -783,10 +858,25 @@ struct Solver {
     for (int k = 0; k < 3; ++k)
       for (int i = t.tid; i < Ms[k]->nls; i += t.T)
         t.slices[Ms[k]->lslot * kWave + i] = ((const int2*)Ms[k]->lsl)[i];
+    for (int j = t.tid; j < p.A.nlong; j += t.T) {
+      const int r = p.A.longs[j], s = p.A.rp[r];
+      t.longs[j] = make_int4(r, p.A.loff ? p.A.loff[j] : 0, s, p.A.rp[r + 1] - s);
+    }
     t.sync();
   }
   // y = M x (FP64); caller syncs before reading y
   __device__ __forceinline__ void spmv(const BCsr& M, const double* __restrict__ x, double* __restrict__ y) {
+    if constexpr (MODE == kLanes) {
+      // x through LDS (at most kLaneMaxRows values; earlier readers of the LDS first)
+      const lptr<double> xl = (lptr<double>)(double*)t.lds;
+      const gptr<const double> xg = (gptr<const double>)x;
+      t.sync();
+      team_each(t, M.lslot == 2 ? p.m : p.n, [=](int i) { return xg[i]; }, [=](int i, double v) { xl[i] = v; });
+      t.sync();
+      rows<double>(
+          M, [=](double v, int c) { return v * xl[c]; }, [=](int r, double s) { y[r] = s; });
+      return;
+    }
     rows<double>(
         M, [=](double v, int c) { return v * x[c]; }, [=](int r, double s) { y[r] = s; });
   }
@@ -964,12 +1054,25 @@ struct Solver {
       const unsigned char* __restrict__ goff = M.goff;
       int* __restrict__ gci = M.gci;
       double* __restrict__ gval = M.gval;
+      if (M.lv32) {
+        // long row j: entries loff[j] + q, q below its padded length
+        unsigned short* __restrict__ lci16 = M.lci16;
+        float* __restrict__ lv32 = M.lv32;
+        for (int j = 0; j < M.nlong; ++j) {
+          const int r = M.longs[j], s = M.loff[j], len = rp[r + 1] - rp[r], pad = M.loff[j + 1] - s;
+          for (int q = t.tid; q < pad; q += t.T) {
+            lci16[s + q] = q < len ? (unsigned short)ci[rp[r] + q] : (unsigned short)0;
+            lv32[s + q] = q < len ? (float)val[rp[r] + q] : 0.f;
+          }
+        }
+      }
       if constexpr (MODE == kLanes) {
         // the lane rows' columns and values
         for (int w = t.tid; w < M.nls * kWave; w += t.T) {
           const int r = w;
           const int at = M.lsl[2 * (w / kWave)] + w % kWave, steps = M.lsl[2 * (w / kWave) + 1];
-          const int s0 = r < M.rows ? rp[r] : 0, len = r < M.rows ? rp[r + 1] - s0 : 0, c0 = r < M.rows ? M.lc0[r] : 0;
+          const int s0 = r < M.rows ? rp[r] : 0, c0 = r < M.rows ? M.lc0[r] : 0;
+          const int len = c0 > 0 ? rp[r + 1] - s0 : 0;  // a long row: none
           const unsigned short first = len > 0 ? (unsigned short)ci[s0] : (unsigned short)0;
           for (int k = 0; k < steps; ++k) {
             const int g = k / kGroupPer, q = g == 0 ? k : c0 + (g - 1) * kGroupPer + k % kGroupPer;
@@ -988,18 +1091,6 @@ struct Solver {
         const int e = r >= 0 ? rp[r] + goff[i] : 0;
         gci[i] = r >= 0 ? ci[e] : 0;
         gval[i] = r >= 0 ? val[e] : 0.0;
-      }
-      if (M.lv32) {
-        // long row j: entries loff[j] + q, q below its padded length
-        unsigned short* __restrict__ lci16 = M.lci16;
-        float* __restrict__ lv32 = M.lv32;
-        for (int j = 0; j < M.nlong; ++j) {
-          const int r = M.longs[j], s = M.loff[j], len = rp[r + 1] - rp[r], pad = M.loff[j + 1] - s;
-          for (int q = t.tid; q < pad; q += t.T) {
-            lci16[s + q] = q < len ? (unsigned short)ci[rp[r] + q] : (unsigned short)0;
-            lv32[s + q] = q < len ? (float)val[rp[r] + q] : 0.f;
-          }
-        }
       }
       if (M.ev32) {
         // slice s, lane l: entries q < the slice's width at
@@ -1041,6 +1132,38 @@ struct Solver {
     t.sync();
   }
 
+  // the tolerance of a solve whose A x64 is not at hand, and its residual:
+  // rhs64 = b1 + A'(rho o b2), r64 = K x64 - rhs64
+  __device__ __forceinline__ double full_residual(const double* b1, const double* b2, int admm_iter) {
+    const int n = p.n, m = p.m;
+    const gptr<const double> rho = (gptr<const double>)p.rho;
+    const gptr<double> x64 = (gptr<double>)p.x64, rhs64 = (gptr<double>)p.rhs64, w64 = (gptr<double>)p.w64;
+    const gptr<const double> gb1 = (gptr<const double>)b1, gb2 = (gptr<const double>)b2;
+    const BCsr &A = p.A, &At = p.At;
+    double eps;
+    // rhs64 = b1 + A'(rho o b2); ||rhs64||_inf
+    rows<double>(
+        At, [=](double v, int c) { return v * (rho[c] * gb2[c]); },
+        [=](int row, double s) { rhs64[row] = gb1[row] + s; });
+    t.sync();
+    const double rhs_norm = norm_inf(p.rhs64, n);
+    if (admm_iter == 1) {
+      S.cg_red_factor = p.set.cg_tol_fraction;
+      S.cg_eps_prev = (rhs_norm < kCgTolMin) ? 1.0 : rhs_norm * S.cg_red_factor;
+      eps = S.cg_eps_prev;
+    } else {
+      eps = next_tolerance();
+    }
+    // w64 = rho o (A x64); r64 = sigma x64 + P x64 + A' w64 - rhs64
+    if (m) {
+      rows<double>(
+        A, [=](double v, int c) { return v * x64[c]; }, [=](int row, double s) { w64[row] = rho[row] * s; });
+      t.sync();
+    }
+    residual64(p.rhs64);
+    return eps;
+  }
+
   // ---- PCG with FP64 defect correction (one linear solve) ----------------------
   // b = [b1 (n); b2 (m)] in/out: out = [x~ ; A x~]
   __device__ __forceinline__ void linsys_solve(double* __restrict__ b1, double* __restrict__ b2, int admm_iter) {
@@ -1066,26 +1189,7 @@ struct Solver {
     const bool cached = m > 0 && S.ax_valid && admm_iter > 1;
     double eps;
     if (!cached) {
-      // rhs64 = b1 + A'(rho o b2); ||rhs64||_inf
-      rows<double>(
-          At, [=](double v, int c) { return v * (rho[c] * gb2[c]); },
-          [=](int row, double s) { rhs64[row] = gb1[row] + s; });
-      t.sync();
-      const double rhs_norm = norm_inf(p.rhs64, n);
-      if (admm_iter == 1) {
-        S.cg_red_factor = p.set.cg_tol_fraction;
-        S.cg_eps_prev = (rhs_norm < kCgTolMin) ? 1.0 : rhs_norm * S.cg_red_factor;
-        eps = S.cg_eps_prev;
-      } else {
-        eps = next_tolerance();
-      }
-      // w64 = rho o (A x64); r64 = sigma x64 + P x64 + A' w64 - rhs64
-      if (m) {
-        rows<double>(
-          A, [=](double v, int c) { return v * x64[c]; }, [=](int row, double s) { w64[row] = rho[row] * s; });
-        t.sync();
-      }
-      residual64(p.rhs64);
+      eps = full_residual(b1, b2, admm_iter);
     } else {
       eps = next_tolerance();
       for (int i = t.tid; i < m; i += t.T) w64[i] = rho[i] * (ax64[i] - gb2[i]);
@@ -1210,6 +1314,279 @@ struct Solver {
       t.sync();
       S.ax_valid = 1;
     }
+  }
+  // ---- one ADMM step over the lane rows ----------------------------------------
+  // compute_rhs, the linear solve and the updates of x, z and y with the
+  // arithmetic of linsys_solve and iterate, element for element and sum for
+  // sum, laid out for latency: the vectors that the products gather from
+  // (x64, w64, the CG's p and w) in LDS; r, d, p and M^-1 in the registers of
+  // the lanes that reduce them; the elementwise passes folded into the passes
+  // that hold the same rows (a lane row's lane is the thread of its element);
+  // a barrier a reduction (its LDS words are taken in turn).  The general step
+  // spent its time waiting: FP64 gathers from global memory, reductions through
+  // LDS, seven barriers a CG iteration (now five).  A CG iteration and its share
+  // of the rest, one team of 512 threads alone: 14.4 to 9.5 us on a 1000-asset
+  // portfolio, 18.1 to 15.3 us on a horizon-50 MPC.
+  // LDS: x64 8 n | r64 8 n (CG: K p) | w64 8 m (CG: w) | p (n, CG precision).
+  __device__ __forceinline__ bool lane_fits() const {
+    return (p.n + kRedBlock - 1) / kRedBlock <= kLaneBlocks * t.W &&
+           (16 + sizeof(V)) * (size_t)p.n + 8 * (size_t)p.m <= (size_t)t.lds_bytes;
+  }
+  // reduction blocks of a wavefront: two of FP64's vectors would spill
+  static constexpr int kLaneBlocks = sizeof(V) == 4 ? 2 : 1;
+  static constexpr int kBlockPer = kRedBlock / kWave;  // a block's elements of a lane
+  __device__ __forceinline__ void lane_admm(int admm_iter) {
+    const int n = p.n, m = p.m, W = t.W;
+    const double sg = p.set.sigma, al = p.set.alpha;
+    const int cg_max = p.set.cg_max_iter;
+    const gptr<const double> rho = (gptr<const double>)p.rho, rhoinv = (gptr<const double>)p.rhoinv;
+    const gptr<const double> q = (gptr<const double>)p.q, l = (gptr<const double>)p.l, u = (gptr<const double>)p.u;
+    const gptr<double> x64 = (gptr<double>)p.x64, ax64 = (gptr<double>)p.ax64;
+    const gptr<double> gx = (gptr<double>)x(), gz = (gptr<double>)z(), gy = (gptr<double>)p.y;
+    const gptr<const double> xp = (gptr<const double>)xprev(), zp = (gptr<const double>)zprev();
+    const gptr<double> gdx = (gptr<double>)p.dx, gdy = (gptr<double>)p.dy;
+    const gptr<const V> gdinv = (gptr<const V>)(const V*)p.cdinv;
+    const lptr<double> xs = (lptr<double>)(double*)t.lds, rs = xs + n, ws = rs + n;
+    const lptr<V> kp = (lptr<V>)rs, wv = (lptr<V>)ws, ps = (lptr<V>)(ws + m);
+    const BCsr &A = p.A, &P = p.P, &At = p.At;
+    const bool guard = sizeof(V) == 4;
+    const int nb = (n + kRedBlock - 1) / kRedBlock;
+    int turn = 0;
+    // the blocks' values of lane 0, then their serial sum and maximum
+    auto red_words = [&]() { return t.red + kMaxRedBlocks / 2 + 2 * kMaxTeamWaves * kLaneBlocks * (turn++ & 1); };
+    // body(k, j, i) for this lane's elements i, in block order, and each
+    // block's end(k, block); written out, so that arrays indexed by (k, j) are registers
+    static_assert(kLaneBlocks <= 2 && kBlockPer == 4, "blocks() is written out");
+    auto blocks = [&](auto body, auto end) __attribute__((always_inline)) {
+      auto block = [&](const int k) __attribute__((always_inline)) {
+        const int b = t.wv + k * W, i = b * kRedBlock + t.lane;
+        if (b < nb) {
+          if (i < n) body(k, 0, i);
+          if (i + kWave < n) body(k, 1, i + kWave);
+          if (i + 2 * kWave < n) body(k, 2, i + 2 * kWave);
+          if (i + 3 * kWave < n) body(k, 3, i + 3 * kWave);
+          end(k, b);
+        }
+      };
+      block(0);
+      if constexpr (kLaneBlocks > 1) block(1);
+    };
+    // zero-iteration bookkeeping of the previous solve (cuda_pcg_interface.cu:266-268)
+    if (S.cg_solves > 0) {
+      if (S.cg_iter == 0) S.cg_zero_iters++;
+      else S.cg_zero_iters = 0;
+    }
+    double eps;
+    t.sync();  // earlier readers of the LDS
+    if (S.ax_valid && admm_iter > 1) {
+      // w64 = rho o (A x64 - b2), b2 = z - y / rho
+      struct WIn {
+        double ri, y, z, r, ax;
+      };
+      team_each(
+          t, m, [=](int i) { return WIn{rhoinv[i], gy[i], zp[i], rho[i], ax64[i]}; },
+          [=](int i, const WIn& v) {
+            const double b2 = (-1.0) * (v.ri * v.y) + 1.0 * v.z;
+            ws[i] = v.r * (v.ax - b2);
+          });
+      team_each(t, n, [=](int i) { return x64[i]; }, [=](int i, double v) { xs[i] = v; });
+      t.sync();
+      // r64 = sigma x64 + P x64 + A' w64 - b1, b1 = sigma x - q
+      for (int sl = t.wv; sl < P.nls; sl += W) {
+        const int row = sl * kWave + t.lane, rr = row < n ? row : 0;
+        const double xv = xp[rr], qv = q[rr];
+        const double sp = lane_row<double>(P, lane_slices(P), sl, t.lane, [=](double v, int c) { return v * xs[c]; });
+        const double st = lane_row<double>(At, lane_slices(At), sl, t.lane, [=](double v, int c) { return v * ws[c]; });
+        if (row < n) rs[row] = sg * xs[row] + sp + st - (sg * xv + (-1.0) * qv);
+      }
+      t.sync();
+      eps = next_tolerance();
+    } else {
+      double* __restrict__ b1 = p.xt;
+      double* __restrict__ b2 = p.zt;
+      for (int i = t.tid; i < n; i += t.T) b1[i] = sg * xp[i] + (-1.0) * q[i];
+      for (int i = t.tid; i < m; i += t.T) {
+        const double v = rhoinv[i] * gy[i];
+        b2[i] = (-1.0) * v + 1.0 * zp[i];
+      }
+      t.sync();
+      eps = full_residual(b1, b2, admm_iter);
+      for (int i = t.tid; i < n; i += t.T) {
+        rs[i] = p.r64[i];
+        xs[i] = x64[i];
+      }
+      t.sync();
+    }
+    // ||r64||_inf
+    double rr[kLaneBlocks][kBlockPer];
+    V r[kLaneBlocks][kBlockPer], d[kLaneBlocks][kBlockPer], pv[kLaneBlocks][kBlockPer], di[kLaneBlocks][kBlockPer];
+    double rn = 0.0;
+    {
+      double* w = red_words();
+      double mx = 0.0;
+      blocks(
+          [&](int k, int j, int i) {
+            di[k][j] = gdinv[i];
+            rr[k][j] = rs[i];
+            mx = dmax(mx, fabs(rr[k][j]));
+          },
+          [&](int, int b) {
+            const double v = osqp_hip::wave_max(mx);
+            if (t.lane == 0) w[b] = v;
+            mx = 0.0;
+          });
+      t.sync();
+      for (int b = 0; b < nb; ++b) rn = dmax(rn, w[b]);
+    }
+    S.cg_solves++;
+    const double scale = (rn > 0.0 && isfinite(rn)) ? rn : 1.0;
+    const double eps_cmp = eps / scale;
+    const double inv = 1.0 / scale;
+    // sum of a block's lane terms (Kahan in FP32) and maximum, all blocks
+    KahanAcc<V> acc;
+    double mx = 0.0;
+    auto sum_end = [&](double* w) {
+      return [&, w](int, int b) {
+        const double v = osqp_hip::wave_sum(acc.value());
+        const double x = osqp_hip::wave_max(mx);
+        if (t.lane == 0) {
+          w[b] = v;
+          w[kMaxTeamWaves * kLaneBlocks + b] = x;
+        }
+        acc = KahanAcc<V>();
+        mx = 0.0;
+      };
+    };
+    auto sum_max = [&](const double* w, double* sum, double* max) {
+      t.sync();
+      double a = 0.0, x = 0.0;
+      for (int b = 0; b < nb; ++b) {
+        a += w[b];
+        x = dmax(x, w[kMaxTeamWaves * kLaneBlocks + b]);
+      }
+      *sum = a;
+      *max = x;
+    };
+    // CG on K d = -r64 / scale
+    double rty, rnorm;
+    {
+      double* w = red_words();
+      blocks(
+          [&](int k, int j, int i) {
+            const V ri = (V)(rr[k][j] * inv);
+            const V yi = di[k][j] * ri;
+            r[k][j] = ri;
+            pv[k][j] = -yi;
+            ps[i] = -yi;
+            d[k][j] = (V)0;
+            acc.add(yi * ri);
+            mx = dmax(mx, fabs((double)ri));
+          },
+          sum_end(w));
+      sum_max(w, &rty, &rnorm);
+    }
+    int it = 0;
+    bool go = rnorm > eps_cmp && it < cg_max;
+    if (guard && !(rty > 0.0 && isfinite(rty))) go = false;
+    while (go) {
+      this->template rows_with<V>(
+          A, [=](double v, int c) { return (V)v * ps[c]; }, [=](int row) { return (V)rho[row]; },
+          [=](int row, V s, V rw) { wv[row] = rw * s; });
+      t.sync();
+      // K p = sigma p + P p + A' w, a row of P and the same row of A' by the same lane
+      for (int sl = t.wv; sl < P.nls; sl += W) {
+        const int row = sl * kWave + t.lane;
+        const V sp = lane_row<V>(P, lane_slices(P), sl, t.lane, [=](double v, int c) { return (V)v * ps[c]; });
+        const V st = lane_row<V>(At, lane_slices(At), sl, t.lane, [=](double v, int c) { return (V)v * wv[c]; });
+        if (row < n) kp[row] = (V)sg * ps[row] + sp + st;
+      }
+      t.sync();
+      V kv[kLaneBlocks][kBlockPer];
+      double pkp;
+      {
+        double* w = red_words();
+        blocks(
+            [&](int k, int j, int i) {
+              kv[k][j] = kp[i];
+              acc.add(pv[k][j] * kv[k][j]);
+            },
+            [&](int, int b) {
+              const double v = osqp_hip::wave_sum(acc.value());
+              if (t.lane == 0) w[b] = v;
+              acc = KahanAcc<V>();
+            });
+        t.sync();
+        pkp = 0.0;
+        for (int b = 0; b < nb; ++b) pkp += w[b];
+      }
+      if (guard && !(pkp > 0.0 && isfinite(pkp))) break;
+      const V alpha = (V)(rty / pkp);
+      double rty_new;
+      {
+        double* w = red_words();
+        blocks(
+            [&](int k, int j, int) {
+              d[k][j] += alpha * pv[k][j];
+              const V ri = r[k][j] + alpha * kv[k][j];
+              const V yi = di[k][j] * ri;
+              r[k][j] = ri;
+              acc.add(yi * ri);
+              mx = dmax(mx, fabs((double)ri));
+            },
+            sum_end(w));
+        sum_max(w, &rty_new, &rnorm);
+      }
+      const double beta = rty_new / rty;
+      it++;
+      rty = rty_new;
+      go = rnorm > eps_cmp && it < cg_max;
+      if (guard && !(rty > 0.0 && isfinite(rty))) go = false;
+      if (go) {
+        const V vb = (V)beta;
+        blocks(
+            [&](int k, int j, int i) {
+              pv[k][j] = vb * pv[k][j] - di[k][j] * r[k][j];
+              ps[i] = pv[k][j];
+            },
+            [](int, int) {});
+        t.sync();
+      }
+    }
+    // x64 += scale d; x and its step
+    blocks(
+        [&](int k, int j, int i) {
+          double xi = xs[i];
+          if (it > 0) xi += scale * (double)d[k][j];
+          x64[i] = xi;
+          xs[i] = xi;
+          const double v = al * xi + (1.0 - al) * xp[i];
+          gx[i] = v;
+          gdx[i] = v - xp[i];
+        },
+        [](int, int) {});
+    S.cg_iter = it;
+    S.cg_total += it;
+    t.sync();
+    // A x64, and z, y and its step (update_z, update_y)
+    struct ZIn {
+      double ri, y, z, l, u, r;
+    };
+    rows_with<double>(
+        A, [=](double v, int c) { return v * xs[c]; },
+        [=](int i) { return ZIn{rhoinv[i], gy[i], zp[i], l[i], u[i], rho[i]}; },
+        [=](int i, double s, const ZIn& g) {
+          ax64[i] = s;
+          double v = g.ri * g.y;
+          v += al * s + (1.0 - al) * g.z;
+          v = dmin(dmax(v, g.l), g.u);
+          gz[i] = v;
+          double dyv = al * s + (1.0 - al) * g.z + (-1.0) * v;
+          dyv = dyv * g.r;
+          gdy[i] = dyv;
+          gy[i] = g.y + dyv;
+        });
+    t.sync();
+    S.ax_valid = 1;
   }
   // tolerance of a non-first ADMM iteration (cuda_pcg_interface.cu:46-60)
   __device__ __forceinline__ double next_tolerance() {
@@ -1727,31 +2104,39 @@ struct Solver {
     const double* __restrict__ rhoinv = p.rhoinv;
     const double* __restrict__ l = p.l;
     const double* __restrict__ u = p.u;
-    // compute_rhs
-    for (int i = t.tid; i < n; i += t.T) xt[i] = sigma * xp[i] + (-1.0) * q[i];
-    for (int i = t.tid; i < m; i += t.T) {
-      const double v = rhoinv[i] * y[i];
-      zt[i] = (-1.0) * v + 1.0 * zp[i];
+    bool stepped = false;
+    if constexpr (MODE == kLanes)
+      if (lane_fits()) {
+        lane_admm(iter);
+        stepped = true;
+      }
+    if (!stepped) {
+      // compute_rhs
+      for (int i = t.tid; i < n; i += t.T) xt[i] = sigma * xp[i] + (-1.0) * q[i];
+      for (int i = t.tid; i < m; i += t.T) {
+        const double v = rhoinv[i] * y[i];
+        zt[i] = (-1.0) * v + 1.0 * zp[i];
+      }
+      t.sync();
+      linsys_solve(xt, zt, iter);
+      // update_x, update_z, update_y
+      for (int i = t.tid; i < n; i += t.T) {
+        const double v = a * xt[i] + (1.0 - a) * xp[i];
+        xx[i] = v;
+        dx[i] = v - xp[i];
+      }
+      for (int i = t.tid; i < m; i += t.T) {
+        double v = rhoinv[i] * y[i];
+        v += a * zt[i] + (1.0 - a) * zp[i];  // add_scaled3's increment form (x == a, sca == 1)
+        v = dmin(dmax(v, l[i]), u[i]);
+        zz[i] = v;
+        double dyv = a * zt[i] + (1.0 - a) * zp[i] + (-1.0) * v;
+        dyv = dyv * rho[i];
+        dy[i] = dyv;
+        y[i] = y[i] + dyv;
+      }
+      t.sync();
     }
-    t.sync();
-    linsys_solve(xt, zt, iter);
-    // update_x, update_z, update_y
-    for (int i = t.tid; i < n; i += t.T) {
-      const double v = a * xt[i] + (1.0 - a) * xp[i];
-      xx[i] = v;
-      dx[i] = v - xp[i];
-    }
-    for (int i = t.tid; i < m; i += t.T) {
-      double v = rhoinv[i] * y[i];
-      v += a * zt[i] + (1.0 - a) * zp[i];  // add_scaled3's increment form (x == a, sca == 1)
-      v = dmin(dmax(v, l[i]), u[i]);
-      zz[i] = v;
-      double dyv = a * zt[i] + (1.0 - a) * zp[i] + (-1.0) * v;
-      dyv = dyv * rho[i];
-      dy[i] = dyv;
-      y[i] = y[i] + dyv;
-    }
-    t.sync();
     // time limit (src/osqp_api.c:743-759), before this iteration's checks
     if (p.set.tl_ticks > 0 && t.decide((long long)wall_clock64() - S.t_start >= p.set.tl_ticks)) {
       S.status = kTimeLimit;

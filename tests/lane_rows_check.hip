@@ -48,7 +48,8 @@ static void check(const char* name, const char* blk, size_t total, int rows, int
   for (int w = 0; w < nls * kWave; ++w) {
     const int r = w, at = lsl[2 * (w / kWave)] + w % kWave, steps = lsl[2 * (w / kWave) + 1];
     CHECK(steps == 1 || steps == 2 || steps == 4 || steps == 8 || steps == 16 || steps == 24, "%s: steps %d", name, steps);
-    const int s0 = r < rows ? rp[r] : 0, len = r < rows ? rp[r + 1] - s0 : 0, c0 = r < rows ? lc0[r] : 0;
+    const int s0 = r < rows ? rp[r] : 0, c0 = r < rows ? lc0[r] : 0,
+              len = c0 > 0 ? rp[r + 1] - s0 : 0;
     for (int k = 0; k < steps; ++k) {
       const int g = k / kGroupPer, q = g == 0 ? k : c0 + (g - 1) * kGroupPer + k % kGroupPer;
       const bool in = g == 0 ? k < c0 : q < len;
@@ -71,6 +72,8 @@ static void check(const char* name, const char* blk, size_t total, int rows, int
   for (int c = 0; c < cols; ++c) x[(size_t)c] = (T)std::sin(0.37 * c + 1.0);
   for (int r = 0; r < rows; ++r) {
     const int at = lsl[2 * (r / kWave)] + r % kWave, steps = lsl[2 * (r / kWave) + 1], len = rp[r + 1] - rp[r];
+    CHECK((lc0[r] == 0) == (len > kLongRow), "%s: row %d of %d entries, first piece %d", name, r, len, lc0[r]);
+    if (len > kLongRow) continue;  // a wavefront's, from the long-row list
     T tot = 0;
     for (int g = 0; g < steps; g += kGroupPer) {
       T acc = 0;

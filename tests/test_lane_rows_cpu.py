@@ -32,7 +32,8 @@ def _problems():
     out.append((_short_rows(64, 64, [1, 2, 3, 4], 2), 1))
     out.append((_short_rows(65, 65, [5, 1, 7], 3), 1))
     out.append((_short_rows(257, 300, [2], 4), 0))      # columns without entries
-    out.append((pr.portfolio(500, seed=5), 0))          # long rows
+    out += [(pr.portfolio(n, seed=n), 1) for n in (500, 1000)]  # long rows of A
+    out.append((pr.portfolio(3000, seed=5), 0))         # rows of A' of 18 entries and more
     p = _short_rows(100, 100, [3], 6)
     p["A"] = sp.vstack([p["A"], sp.csc_matrix((1, 100))], format="csc")
     out.append((p, 0))                                  # an empty row
