@@ -211,8 +211,10 @@ void       osqp_amd_linsys_set_w_given(LinSysSolver* s, OSQPInt given);
  * y in place, with delta_x / delta_y of the last one: for small and medium
  * problems, where separate launches cost more than their work.  Returns the
  * iterations queued: `iters`, or 0 when this linsys has no such path or the
- * PCG has no A x to continue from (the caller then iterates as usual). */
-OSQPInt    osqp_amd_linsys_run(LinSysSolver* s, OSQPInt iters, OSQPFloat alpha, OSQPVectorf* x,
+ * PCG has no A x to continue from (the caller then iterates as usual).
+ * eq_rows: some rows are equality constraints; only a path that keeps the
+ * separate kernels' order of summation is then taken. */
+OSQPInt    osqp_amd_linsys_run(LinSysSolver* s, OSQPInt iters, OSQPInt eq_rows, OSQPFloat alpha, OSQPVectorf* x,
                                OSQPVectorf* delta_x, OSQPVectorf* z, OSQPVectorf* y, OSQPVectorf* delta_y,
                                const OSQPVectorf* q, const OSQPVectorf* l, const OSQPVectorf* u,
                                const OSQPVectorf* rho_inv);

@@ -11,6 +11,8 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <stdlib.h>
+
 #include "host_internal.h"
 
 const char* OSQP_STATUS_MESSAGE[] = {"",
@@ -95,6 +97,20 @@ OSQPInt adapt_rho(OSQPSolver* solver) {
   return exitflag;
 }
 
+/* whether a constraint is an equality (its rho is OSQP_RHO_EQ_OVER_RHO_INEQ times
+ * the others'); unknown counts as yes */
+static OSQPInt has_equality(const OSQPVectori* types) {
+  const OSQPInt m = OSQPVectori_length(types);
+  OSQPInt *t, i, found = 0;
+  if (m <= 0) return 0;
+  t = (OSQPInt*)malloc(sizeof(OSQPInt) * (size_t)m);
+  if (!t) return 1;
+  OSQPVectori_to_raw(t, types);
+  for (i = 0; i < m && !found; i++) found = t[i] == 1;
+  free(t);
+  return found;
+}
+
 /* auxil.c:76-105 */
 OSQPInt set_rho_vec(OSQPSolver* solver) {
   OSQPSettings* settings = solver->settings;
@@ -103,6 +119,7 @@ OSQPInt set_rho_vec(OSQPSolver* solver) {
   settings->rho = c_min(c_max(settings->rho, OSQP_RHO_MIN), OSQP_RHO_MAX);
   changed = OSQPVectorf_ew_bounds_type(work->constr_type, work->data->l, work->data->u, OSQP_RHO_TOL,
                                        OSQP_INFTY * OSQP_MIN_SCALING);
+  if (changed) work->eq_rows = has_equality(work->constr_type);
   OSQPVectorf_set_scalar_conditional(work->rho_vec, work->constr_type, OSQP_RHO_MIN, settings->rho,
                                      OSQP_RHO_EQ_OVER_RHO_INEQ * settings->rho);
   OSQPVectorf_ew_reciprocal(work->rho_inv_vec, work->rho_vec);

@@ -44,6 +44,7 @@ struct OSQPWorkspace_ {
   OSQPVectorf*  rho_vec;
   OSQPVectorf*  rho_inv_vec;
   OSQPVectori*  constr_type;
+  OSQPInt       eq_rows;       /* constr_type holds equality constraints */
   OSQPVectorf *x, *y, *z, *xz_tilde, *xtilde_view, *ztilde_view, *x_prev, *z_prev;
   OSQPVectorf *Ax, *Px, *Aty;
   OSQPFloat    xtPx, qtx, SC, scaled_dual_gap;

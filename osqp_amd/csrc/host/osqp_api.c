@@ -434,7 +434,7 @@ OSQPInt osqp_solve(OSQPSolver* solver) {
   for (iter = 1; iter <= settings->max_iter; iter++) {
     OSQPInt ran = free_iterations(solver, iter);
     if (ran > 0)
-      ran = osqp_amd_linsys_run(work->linsys_solver, ran, settings->alpha, work->x, work->delta_x, work->z, work->y,
+      ran = osqp_amd_linsys_run(work->linsys_solver, ran, work->eq_rows, settings->alpha, work->x, work->delta_x, work->z, work->y,
                                 work->delta_y, work->data->q, work->data->l, work->data->u, work->rho_inv_vec);
     if (ran > 0) {
       iter += ran - 1;

@@ -129,3 +129,18 @@ def test_rows_out_of_order_stay_on_the_separate_kernels():
         s.close()
     assert r["sorted"].info.status_val == r["reversed"].info.status_val == 1
     assert np.linalg.norm(r["sorted"].x - r["reversed"].x) <= 1e-3 * np.linalg.norm(r["sorted"].x)
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("features", [500, 620])
+def test_equality_rows_keep_the_separate_kernels_order(features, precision):
+    """A lasso's equality rows (too many entries for one workgroup): the same bits as the separate kernels;
+    relaxed to inequalities, the several-workgroup kernel's solve ends at a certified point."""
+    p = pr.lasso(features, 10 * features + 3, 0.02, seed=features)
+    relaxed = dict(l=p["l"] - 0.05, u=p["u"] + 0.05)
+    a, b = both(p, precision, second=relaxed, **EPS)
+    assert a[0][2:] == b[0][2:]
+    assert np.array_equal(a[0][0], b[0][0]) and np.array_equal(a[0][1], b[0][1])
+    assert a[1][3] == b[1][3] == 1
+    c = pr.kkt_certificate(dict(p, **relaxed), b[1][0], b[1][1])
+    assert c["prim"] <= 1e-4 + 1e-4 * c["scale_p"] and c["dual"] <= 1e-4 + 1e-4 * c["scale_d"]
