@@ -65,7 +65,7 @@ void download(void* dst, const void* src, size_t bytes);  // host or device dst;
 // v_permlane32_swap / v_permlane16_swap, the rest by row rotations (lanes that
 // a rotation pairs hold the values that the xor would pair).  Register moves
 // only: a step through LDS (ds_bpermute) costs its latency, in a chain of six.
-// Nine reductions and three products of 8000 x 80001: 155 to 147 us.
+// Nine reductions and three products of 8000 x 80001: 153 to 151 us (147 in another run).
 template <typename T, typename F>
 __device__ __forceinline__ T lane_words(T v, F f) {
   static_assert(sizeof(T) == 4 || sizeof(T) == 8, "4 or 8 bytes");
