@@ -218,6 +218,19 @@ OSQPInt    osqp_amd_linsys_run(LinSysSolver* s, OSQPInt iters, OSQPInt eq_rows, 
                                OSQPVectorf* delta_x, OSQPVectorf* z, OSQPVectorf* y, OSQPVectorf* delta_y,
                                const OSQPVectorf* q, const OSQPVectorf* l, const OSQPVectorf* u,
                                const OSQPVectorf* rho_inv);
+/* Whether the last osqp_amd_linsys_run gave up on the device: its workgroups
+ * wait for each other, and a wait that lasts too long (a workgroup that never
+ * got onto the GPU) ends the launch.  1: x, z, y and the solver's state are
+ * again what they were before that run, delta_x and delta_y are undefined, and
+ * the path is off from then on.  To be asked after each run, before its
+ * results are used and before the next one; `waited`: the caller has already
+ * received a result queued after the run, so there is nothing to wait for. */
+OSQPInt    osqp_amd_linsys_run_failed(LinSysSolver* s, OSQPInt waited);
+/* ADMM iterations done by osqp_amd_linsys_run, its workgroups (0: the path is
+ * off) and the runs that gave up or were refused. */
+OSQPInt    osqp_amd_linsys_run_stats(LinSysSolver* s, long long* iters, OSQPInt* groups, OSQPInt* failed);
+/* Looks after which a workgroup's wait gives up, for this solver (checks). */
+void       osqp_amd_linsys_run_polls(LinSysSolver* s, OSQPInt polls);
 /* Queued reductions (no counterpart in the reference, whose reductions each
  * return to the host): each call queues the same reduction as
  * OSQPVectorf_norm_inf / scaled_norm_inf / dot_prod / dot_prod_signed (same

@@ -846,8 +846,13 @@ struct HipPcg {
   float* ap;
   float* u;
   int z_incr, z_count, z_use;
-  // the whole loop in one launch, for small and medium problems (runner.h)
+  // the whole loop in one launch, for small and medium problems (runner.h);
+  // a launch of several workgroups whose result is not yet known, and what the
+  // host counted before it
   Runner run;
+  RunCall run_call;
+  int run_open, run_solves, run_z_count, run_failed;
+  long long run_iters;  // ADMM iterations the runner has done
 };
 
 // solves between two exact recomputations of the cached A x64
@@ -1494,10 +1499,11 @@ OSQPInt pcg_solve(LinSysSolver* self, OSQPVectorf* b, OSQPInt admm_iter) {
     s->h_flags = nullptr;
     s->d_flags = nullptr;
     s->flags_len = 0;
-    if (hipHostMalloc((void**)&s->h_flags, sizeof(int) * (size_t)(s->max_iter + 1),
+    // a flag per CG iteration, then the runner's word (run_word)
+    if (hipHostMalloc((void**)&s->h_flags, sizeof(int) * (size_t)(s->max_iter + 2),
                       hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess &&
         hipHostGetDevicePointer((void**)&s->d_flags, s->h_flags, 0) == hipSuccess) {
-      memset(s->h_flags, 0, sizeof(int) * (size_t)(s->max_iter + 1));
+      memset(s->h_flags, 0, sizeof(int) * (size_t)(s->max_iter + 2));
       s->flags_len = s->max_iter + 1;
     } else {
       (void)hipGetLastError();
@@ -1670,7 +1676,8 @@ OSQPInt osqp_algebra_init_linsys_solver(LinSysSolver** sp, const OSQPMatrix* P, 
   // The runner multiplies by CG-precision copies throughout: with the FP32 CG
   // only where the defect correction reads FP32 copies anyway.
   const bool copies = s->bits == 64 || (s->dcK32 && s->dcA32);
-  if (!polishing && rho_vec && copies && runner_build(&s->run, A, P, RunK{s->krp, s->kci, s->kval64}, s->bits)) {
+  if (!polishing && rho_vec && copies && runner_build(&s->run, A, P, RunK{s->krp, s->kci, s->kval64}, s->bits,
+                                                     sizeof(PcgState) / sizeof(double))) {
     pcg_free(&s->base);
     *sp = nullptr;
     return OSQP_LINSYS_SOLVER_INIT_ERROR;
@@ -1692,9 +1699,11 @@ OSQPInt osqp_amd_linsys_run(LinSysSolver* ls, OSQPInt iters, OSQPInt eq_rows, OS
                             const OSQPVectorf* rho_inv) {
   HipPcg* s = (HipPcg*)ls;
   if (!s || !s->run.on || iters <= 0 || s->polishing || !s->rho_vec || (eq_rows && s->run.G > 1)) return 0;
+  if (!s->h_flags || s->run_open) return 0;
   if (!s->ax_valid || s->ax_Aver != s->A->version) return 0;  // the first iteration builds A x64
   if (s->kver_P != s->P->version || s->kver_A != s->A->version || (s->bits == 32 && s->A->fp32_dirty))
     update_precond(s);
+  static_assert(sizeof(PcgState) % sizeof(double) == 0, "the state is saved as doubles");
   RunCall c;
   c.iters = iters;
   c.z_count = s->z_count;
@@ -1721,10 +1730,55 @@ OSQPInt osqp_amd_linsys_run(LinSysSolver* ls, OSQPInt iters, OSQPInt eq_rows, OS
   PcgState* st = s->st;
   c.st = RunState{&st->eps_prev, &st->red_factor, &st->zero_iters, &st->iter, &st->solves, &st->active, &st->done,
                   &st->total_iters};
-  s->z_count = runner_run(&s->run, s->A, s->P, RunK{s->krp, s->kci, s->kval64}, c);
+  c.state = (double*)st;
+  c.bad = s->d_flags + s->flags_len;
+  int z_count = 0;
+  if (runner_run(&s->run, s->A, s->P, RunK{s->krp, s->kci, s->kval64}, c, &z_count)) {
+    s->run.on = 0;
+    s->run_failed++;
+    return 0;
+  }
+  s->run_open = s->run.G > 1;
+  s->run_call = c;
+  s->run_solves = s->host_solves;
+  s->run_z_count = s->z_count;
+  s->z_count = z_count;
   s->host_solves += iters;
+  s->run_iters += iters;
   s->w_given = 0;
   return iters;
+}
+
+OSQPInt osqp_amd_linsys_run_failed(LinSysSolver* ls, OSQPInt waited) {
+  HipPcg* s = (HipPcg*)ls;
+  if (!s || !s->run_open) return 0;
+  s->run_open = 0;
+  if (!waited) HIPCHK(hipStreamSynchronize(S()));
+  volatile int* bad = (volatile int*)s->h_flags + s->flags_len;
+  if (!*bad) return 0;
+  HIPCHK(hipStreamSynchronize(S()));
+  *bad = 0;
+  runner_restore(&s->run, s->run_call);
+  s->host_solves = s->run_solves;
+  s->z_count = s->run_z_count;
+  s->run_iters -= s->run_call.iters;
+  s->run.on = 0;
+  s->run_failed++;
+  return 1;
+}
+
+OSQPInt osqp_amd_linsys_run_stats(LinSysSolver* ls, long long* iters, OSQPInt* groups, OSQPInt* failed) {
+  HipPcg* s = (HipPcg*)ls;
+  if (!s) return 1;
+  if (iters) *iters = s->run_iters;
+  if (groups) *groups = s->run.on ? s->run.G : 0;
+  if (failed) *failed = s->run_failed;
+  return 0;
+}
+
+void osqp_amd_linsys_run_polls(LinSysSolver* ls, OSQPInt polls) {
+  HipPcg* s = (HipPcg*)ls;
+  if (s && polls >= 0) s->run.polls = polls;
 }
 
 // Times the two CG operator kernels (w = rho o A p and Kp = sigma p + P p + A' w)

@@ -53,6 +53,7 @@ struct RunOp {
 struct Runner {
   int on;             // built and usable
   int n, m, G, bits;
+  int state_len;      // doubles of the PCG's device state
   int cw;             // columns per chunk
   int rows_max;       // rows of the largest workgroup range
   int resident;       // the copies held in LDS
@@ -66,7 +67,8 @@ struct Runner {
   double* part;       // G * n shares
   double* xch;        // 2 n: r64, K p
   unsigned* bar;      // barrier words
-  int* bad;           // a barrier gave up
+  double* save;       // what a launch changes, as it was before it (runner_restore)
+  int polls;          // a barrier's wait gives up after this many looks
   long long ver_A, ver_P;  // versions the values were copied from
 };
 
@@ -91,13 +93,20 @@ struct RunCall {
   double *x64, *ax64;
   const void* dinv;                                 // CG precision
   RunState st;
+  double* state;                                    // the PCG's device state (Runner::state_len)
+  int* bad;           // host-coherent word, set where a barrier gave up
 };
 
 // Builds the runner for A (m x n, CSR and CSC on the device) when it pays and
 // fits; r->on stays 0 otherwise.  Returns 1 on an allocation failure.
-int runner_build(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P, const RunK& k, int bits);
+// state_len: doubles of the PCG's device state.
+int runner_build(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P, const RunK& k, int bits, int state_len);
 void runner_free(Runner* r);
-// Queues c.iters ADMM iterations; returns the new z_count.
-int runner_run(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P, const RunK& k, const RunCall& c);
+// Queues c.iters ADMM iterations and leaves the new z_count; 1 when the launch
+// was refused (nothing has changed then).
+int runner_run(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P, const RunK& k, const RunCall& c, int* z_count);
+// Several workgroups: x, z, y, x64, A x64 and the PCG's state as they were
+// before the last launch.
+void runner_restore(Runner* r, const RunCall& c);
 
 }  // namespace osqp_hip

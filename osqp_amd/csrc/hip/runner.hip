@@ -20,6 +20,7 @@ constexpr int kRunRefresh = 8;      // ADMM iterations between two exact recompu
 constexpr uint16_t kNoRow = 0xFFFF;
 constexpr size_t kRunLds = 159 * 1024;  // dynamic LDS of a launch
 constexpr long long kRun1Work = 48000;  // entries of A and P up to which one workgroup runs alone
+constexpr int kRunPolls = 1 << 22;  // looks of a barrier's wait, some seconds
 
 inline hipStream_t S() { return rt().stream; }
 
@@ -198,15 +199,17 @@ struct RunArgs {
   RunView A, At, P, A2;
   double *part, *xch;
   unsigned* bar;
-  int* bad;
+  int polls;
   RunCall c;
 };
 
 // Grid barrier of workgroups that are all resident (cooperative launch), in
 // two levels: 8 groups of workgroups (blockIdx mod 8, an XCD each in dispatch
 // order), then the groups.  Words 64 apart.  Every wavefront's stores have
-// completed (vmcnt) before its workgroup arrives.  The wait is bounded: past
-// it the workgroup marks `bad` and every workgroup leaves the kernel.
+// completed (vmcnt) before its workgroup arrives.  The wait is bounded (polls):
+// past it the workgroup sets the host's word and leaves the kernel, as the
+// others do at their next barrier; the host then restores what the launch
+// changed (runner_restore).
 __device__ __forceinline__ bool grid_barrier(const RunArgs& a, unsigned epoch, int* flag) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
@@ -219,8 +222,9 @@ __device__ __forceinline__ bool grid_barrier(const RunArgs& a, unsigned epoch, i
         for (unsigned k = 0; k < ng; ++k) stx(w + (9 + k) * 64, epoch);
     }
     for (int k = 0; ldx(w + (9 + g) * 64) < epoch; ++k) {
-      if (k > (1 << 22)) {
-        stx(a.bad, 1);
+      if (k >= a.polls) {
+        __hip_atomic_store(a.c.bad, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // with the host before this launch ends
         ok = 0;
         break;
       }
@@ -1069,6 +1073,27 @@ __global__ void k_zero_words(unsigned* p, int k) {
 
 constexpr int kBarWords = 17 * 64;
 
+// What a launch of several workgroups changes in place, copied before it (and
+// back when it gave up): x, x64, z, y, A x64 and the PCG's state.  With
+// delta x and delta y, which a later iteration writes whole, that is all.
+size_t run_save_len(int n, int m, int state_len) { return 2 * (size_t)n + 3 * (size_t)m + (size_t)state_len; }
+__global__ void k_run_save(int n, int m, int state_len, RunCall c, double* save, int back) {
+  const long long total = 2LL * n + 3LL * m + state_len;
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < total;
+       i += (long long)gridDim.x * blockDim.x) {
+    long long k = i;
+    double* p;
+    if (k < n) p = c.x + k;
+    else if ((k -= n) < n) p = c.x64 + k;
+    else if ((k -= n) < m) p = c.z + k;
+    else if ((k -= m) < m) p = c.y + k;
+    else if ((k -= m) < m) p = c.ax64 + k;
+    else p = c.state + (k - m);
+    if (back) *p = save[i];
+    else save[i] = *p;
+  }
+}
+
 // copies in LDS: n up to 4 kT (runner_build)
 template <typename V, int NE>
 const void* run_kernel(bool res) {
@@ -1303,6 +1328,7 @@ void runner_free(Runner* r) {
   dev_free(r->part);
   dev_free(r->xch);
   dev_free(r->bar);
+  dev_free(r->save);
   memset(r, 0, sizeof(*r));
 }
 
@@ -1342,9 +1368,9 @@ static int build_many(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P) {
   }
   r->part = (double*)dev_alloc(sizeof(double) * (size_t)G * n);
   r->xch = (double*)dev_alloc(sizeof(double) * 2 * (size_t)n);
-  r->bar = (unsigned*)dev_alloc(sizeof(unsigned) * (kBarWords + 64));
-  if (alloc_op(r, &r->A) || alloc_op(r, &r->At) || alloc_op(r, &r->P) || !r->part || !r->xch || !r->bar) return 1;
-  r->bad = (int*)(r->bar + kBarWords);
+  r->bar = (unsigned*)dev_alloc(sizeof(unsigned) * kBarWords);
+  r->save = (double*)dev_alloc(sizeof(double) * run_save_len(n, r->m, r->state_len));
+  if (alloc_op(r, &r->A) || alloc_op(r, &r->At) || alloc_op(r, &r->P) || !r->part || !r->xch || !r->bar || !r->save) return 1;
   fill_A(r, A, true);
   fill_P(r, P, true);
   const size_t copies = ((size_t)r->A.max_steps + r->At.max_steps + r->P.max_steps) * kWave * ((size_t)r->bits / 8 + 2);
@@ -1352,11 +1378,10 @@ static int build_many(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P) {
     r->resident = 1;
     r->lds += copies;
   }
-  hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(kBlock), 0, S(), r->bar, kBarWords + 64);
   return 0;
 }
 
-int runner_build(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P, const RunK& k, int bits) {
+int runner_build(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P, const RunK& k, int bits, int state_len) {
   memset(r, 0, sizeof(*r));
   const int n = A->n, m = A->m;
   if (A->is_triu || n <= 0 || m <= 0 || A->nnz <= 0 || n > run_n_max(bits)) return 0;
@@ -1382,6 +1407,8 @@ int runner_build(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P, const RunK
     r->m = m;
     r->bits = bits;
     r->G = G;
+    r->state_len = state_len;
+    r->polls = kRunPolls;
     rc = build_many(r, A, P);
   }
   if (rc || r->G == 0) {
@@ -1396,7 +1423,15 @@ int runner_build(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P, const RunK
   return 0;
 }
 
-int runner_run(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P, const RunK& k, const RunCall& c) {
+static void run_save(const Runner* r, const RunCall& c, int back) {
+  const int g = grid_for((long long)run_save_len(r->n, r->m, r->state_len), kBlock, 1024);
+  hipLaunchKernelGGL(k_run_save, dim3(g), dim3(kBlock), 0, S(), r->n, r->m, r->state_len, c, r->save, back);
+}
+void runner_restore(Runner* r, const RunCall& c) {
+  run_save(r, c, 1);
+}
+
+int runner_run(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P, const RunK& k, const RunCall& c, int* z_count) {
   const bool many = r->G > 1;
   if (many) {
     if (r->ver_A != A->version) fill_A(r, A, false);
@@ -1420,19 +1455,25 @@ int runner_run(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P, const RunK& 
   a.part = r->part;
   a.xch = r->xch;
   a.bar = r->bar;
-  a.bad = r->bad;
+  a.polls = r->polls;
   a.c = c;
   void* args[] = {&a};
+  hipError_t err;
   if (many) {
+    run_save(r, c, 0);
     hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(kBlock), 0, S(), r->bar, kBarWords);
-    HIPCHK(hipLaunchCooperativeKernel(kernel_of(r), dim3(r->G), dim3(kT), args, (unsigned)r->lds, S()));
+    err = hipLaunchCooperativeKernel(kernel_of(r), dim3(r->G), dim3(kT), args, (unsigned)r->lds, S());
   } else {
-    HIPCHK(hipLaunchKernel(kernel_of(r), dim3(1), dim3(kT), args, r->lds, S()));
-    if (r->bits == 64) return c.z_count;  // A x64 is exact in every iteration
+    err = hipLaunchKernel(kernel_of(r), dim3(1), dim3(kT), args, r->lds, S());
   }
-  int zc = c.z_count;
-  for (int i = 0; i < c.iters; ++i) zc = zc >= kRunRefresh - 1 ? 0 : zc + 1;
-  return zc;
+  if (err != hipSuccess) {
+    (void)hipGetLastError();
+    return 1;
+  }
+  *z_count = c.z_count;
+  if (!many && r->bits == 64) return 0;  // A x64 is exact in every iteration
+  for (int i = 0; i < c.iters; ++i) *z_count = *z_count >= kRunRefresh - 1 ? 0 : *z_count + 1;
+  return 0;
 }
 
 }  // namespace osqp_hip

@@ -432,7 +432,9 @@ OSQPInt osqp_solve(OSQPSolver* solver) {
   work->rhs_ready = 0;
 
   for (iter = 1; iter <= settings->max_iter; iter++) {
-    OSQPInt ran = free_iterations(solver, iter);
+    OSQPInt ran = free_iterations(solver, iter), checked;
+    const OSQPInfo info_before = *solver->info;
+    const OSQPFloat prim_before = work->scaled_prim_res, dual_before = work->scaled_dual_res;
     if (ran > 0)
       ran = osqp_amd_linsys_run(work->linsys_solver, ran, work->eq_rows, settings->alpha, work->x, work->delta_x, work->z, work->y,
                                 work->delta_y, work->data->q, work->data->l, work->data->u, work->rho_inv_vec);
@@ -467,6 +469,7 @@ OSQPInt osqp_solve(OSQPSolver* solver) {
   iterated:
     /* src/osqp_api.c:728-737 */
     if (osqp_amd_interrupted()) {
+      if (ran > 0) osqp_amd_linsys_run_failed(work->linsys_solver, 0);
       update_status(solver->info, OSQP_SIGINT);
       if (settings->verbose) printf("Solver interrupted\n");
       exitflag = 1;
@@ -476,6 +479,7 @@ OSQPInt osqp_solve(OSQPSolver* solver) {
     if (work->first_run) temp_run_time = solver->info->setup_time + osqp_amd_toc(work);
     else temp_run_time = solver->info->update_time + osqp_amd_toc(work);
     if (settings->time_limit && (temp_run_time >= settings->time_limit)) {
+      if (ran > 0) osqp_amd_linsys_run_failed(work->linsys_solver, 0);
       update_status(solver->info, OSQP_TIME_LIMIT_REACHED);
       can_print = 0;
       break;
@@ -509,7 +513,16 @@ OSQPInt osqp_solve(OSQPSolver* solver) {
         break;
     }
 
-    if (can_check || can_print || can_adapt || iter == 1) update_info(solver, iter);
+    checked = can_check || can_print || can_adapt || iter == 1;
+    if (checked) update_info(solver, iter);
+    if (ran > 0 && osqp_amd_linsys_run_failed(work->linsys_solver, checked)) {
+      /* again from where the run began, on the separate kernels */
+      *solver->info = info_before;
+      work->scaled_prim_res = prim_before;
+      work->scaled_dual_res = dual_before;
+      iter -= ran;
+      continue;
+    }
     if (can_check && check_termination(solver, 0)) break;
 
     work->rho_updated = 0;
@@ -839,6 +852,17 @@ OSQPInt osqp_amd_solver_stats(OSQPSolver* solver, OSQPInt* pcg_iters_total, OSQP
   if (!solver || !solver->work || !solver->work->linsys_solver) return 1;
   osqp_amd_linsys_counters(solver->work->linsys_solver, pcg_iters_total, linsys_solves);
   if (gpu_ms) *gpu_ms = solver->info->solve_time * 1e3;
+  return 0;
+}
+
+OSQPInt osqp_amd_solver_run_stats(OSQPSolver* solver, long long* iters, OSQPInt* groups, OSQPInt* failed) {
+  if (!solver || !solver->work || !solver->work->linsys_solver) return 1;
+  return osqp_amd_linsys_run_stats(solver->work->linsys_solver, iters, groups, failed);
+}
+
+OSQPInt osqp_amd_solver_run_polls(OSQPSolver* solver, OSQPInt polls) {
+  if (!solver || !solver->work || !solver->work->linsys_solver || polls < 0) return 1;
+  osqp_amd_linsys_run_polls(solver->work->linsys_solver, polls);
   return 0;
 }
 

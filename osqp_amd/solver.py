@@ -62,6 +62,11 @@ def load_library():
         lib.osqp_amd_solver_stats.argtypes = [C.POINTER(T.OSQPSolver), C.POINTER(C.c_int), C.POINTER(C.c_int),
                                               C.POINTER(C.c_double)]
         lib.osqp_amd_solver_stats.restype = C.c_int
+        lib.osqp_amd_solver_run_stats.argtypes = [C.POINTER(T.OSQPSolver), C.POINTER(C.c_longlong),
+                                                  C.POINTER(C.c_int), C.POINTER(C.c_int)]
+        lib.osqp_amd_solver_run_stats.restype = C.c_int
+        lib.osqp_amd_solver_run_polls.argtypes = [C.POINTER(T.OSQPSolver), C.c_int]
+        lib.osqp_amd_solver_run_polls.restype = C.c_int
         lib.osqp_amd_apply_operator.argtypes = [C.POINTER(T.OSQPSolver), C.c_int, vp, vp]
         lib.osqp_amd_apply_operator.restype = C.c_int
         lib.osqp_amd_time_pcg_kernels.argtypes = [C.POINTER(T.OSQPSolver), C.c_int] + [C.POINTER(C.c_double)] * 4
@@ -235,6 +240,18 @@ class OSQP:
         it, sv, ms = C.c_int(), C.c_int(), C.c_double()
         self.lib.osqp_amd_solver_stats(self._solver, C.byref(it), C.byref(sv), C.byref(ms))
         return SimpleNamespace(pcg_iters=it.value, linsys_solves=sv.value, solve_ms=ms.value)
+
+    def run_stats(self):
+        """ADMM iterations that ran many to a launch, that launch's workgroups
+        (0: the path is off) and the launches that gave up or were refused."""
+        it, g, f = C.c_longlong(), C.c_int(), C.c_int()
+        self.lib.osqp_amd_solver_run_stats(self._solver, C.byref(it), C.byref(g), C.byref(f))
+        return SimpleNamespace(iters=it.value, groups=g.value, failed=f.value)
+
+    def run_polls(self, polls):
+        """Looks after which such a launch's waits give up (checks)."""
+        if self.lib.osqp_amd_solver_run_polls(self._solver, int(polls)):
+            raise ValueError("polls must not be negative")
 
     def apply_operator(self, which, x):
         """The linear system's operator on x through its own kernels:

@@ -112,6 +112,38 @@ def test_many_workgroups_fp32(n, m, row):
             assert c["dual"] <= 1e-4 + 1e-4 * c["scale_d"]
 
 
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("check", [25, 0])
+def test_a_wait_that_gives_up_is_done_again(precision, check):
+    """Waits that give up at once (every workgroup leaves its launch): the iterations of that launch are
+    done again by the separate kernels, so the solve and the next one are theirs to the bit."""
+    p = qp(700, 9001, 30, seed=9)
+    # without checks and rho updates the host sees nothing of a run but whether it gave up
+    st = dict(EPS, check_termination=check, **({} if check else dict(adaptive_rho=0, max_iter=100)))
+    out = []
+    for polls in (None, 0):
+        s = OSQP(precision=precision)
+        assert s.setup(p["P"], p["q"], p["A"], p["l"], p["u"], profiler_level=1 if polls is None else 0, **st) == 0
+        if polls is not None:
+            assert s.run_stats().groups > 1
+            s.run_polls(polls)
+        r = []
+        for q in (p["q"], p["q2"]):
+            s.update(q=q)
+            r.append(s.solve())
+            assert r[-1].rc == 0
+        out.append((r, s.stats().pcg_iters, s.run_stats()))
+        s.close()
+    (a, na, sa), (b, nb, sb) = out
+    assert (sa.iters, sa.failed) == (0, 0) and (sb.iters, sb.failed, sb.groups) == (0, 1, 0)
+    assert na == nb
+    for u, v in zip(a, b):
+        assert (u.info.iter, u.info.status_val) == (v.info.iter, v.info.status_val)
+        assert np.array_equal(u.x, v.x) and np.array_equal(u.y, v.y)
+        for f in ("prim_res", "dual_res", "obj_val", "primdual_int", "rho_updates"):
+            assert getattr(u.info, f) == getattr(v.info, f)
+
+
 def test_rows_out_of_order_stay_on_the_separate_kernels():
     """Columns whose rows are not ascending: the several-workgroup layout needs the order, so the solve
     takes the separate kernels and gives the sorted problem's answer."""
