@@ -1690,15 +1690,24 @@ OSQPInt osqp_algebra_init_linsys_solver(LinSysSolver** sp, const OSQPMatrix* P, 
 // on that order: of 40 lassos with 500..680 features in FP64, 11 ended with an
 // error against the exact optimum more than 1.1 times the separate kernels'
 // (FP32, 500..1020 features: 4 of 40), while random QPs of inequalities kept
-// theirs.  So with equality rows only the one-workgroup kernel, whose sums are
-// the separate kernels', takes the loop; a lasso of 10001 features stays at
-// 225 ms (173 ms with sums in another order).
+// theirs.  So with equality rows the loop is run in one launch only where its
+// sums are the separate kernels': by one workgroup, and with every operator one
+// column panel (n + m <= 4096).  Past one panel those kernels add a row panel
+// by panel, the one workgroup does not: an MPC of horizon 110 (n + m = 4876)
+// takes 148 us an ADMM iteration on them, 72 in one launch.
+static bool one_panel(const HipPcg* s) {
+  const auto one = [](const PanelMatrix* P) { return P && P->np == 1; };
+  return one(panels_A<double>(s)) && one(panels_K<double>(s)) &&
+         (s->bits == 64 || (one(panels_A<float>(s)) && one(panels_K<float>(s))));
+}
+
 OSQPInt osqp_amd_linsys_run(LinSysSolver* ls, OSQPInt iters, OSQPInt eq_rows, OSQPFloat alpha, OSQPVectorf* x,
                             OSQPVectorf* delta_x, OSQPVectorf* z, OSQPVectorf* y, OSQPVectorf* delta_y,
                             const OSQPVectorf* q, const OSQPVectorf* l, const OSQPVectorf* u,
                             const OSQPVectorf* rho_inv) {
   HipPcg* s = (HipPcg*)ls;
-  if (!s || !s->run.on || iters <= 0 || s->polishing || !s->rho_vec || (eq_rows && s->run.G > 1)) return 0;
+  if (!s || !s->run.on || iters <= 0 || s->polishing || !s->rho_vec) return 0;
+  if (eq_rows && (s->run.G > 1 || !one_panel(s))) return 0;
   if (!s->h_flags || s->run_open) return 0;
   if (!s->ax_valid || s->ax_Aver != s->A->version) return 0;  // the first iteration builds A x64
   if (s->kver_P != s->P->version || s->kver_A != s->A->version || (s->bits == 32 && s->A->fp32_dirty))

@@ -675,9 +675,10 @@ __global__ __launch_bounds__(kT) void k_admm_run(RunArgs a) {
 
 // ---- one workgroup ---------------------------------------------------------------
 // The same loop for problems of one workgroup, over A's rows and the rows of
-// K = [P A'] as the column-panel kernels take them: each row on the lanes, in
-// the order and with the epilogue of those kernels, and every dot product in
-// the blocks of theirs, so the iterates are theirs to the bit (their FP32
+// K = [P A'] as the column-panel kernels take them where one panel holds all
+// columns: each row on the lanes, in the order and with the epilogue of those
+// kernels, and every dot product in the blocks of theirs, so the iterates are
+// theirs to the bit, up to n + m of one panel's columns (their FP32
 // rounding decides where a CG stops on problems with tight equality
 // constraints, and the ADMM iterates part after that).  FP64 recomputes A x64
 // in every iteration, as the separate kernels do.
