@@ -218,6 +218,11 @@ OSQPInt    osqp_amd_linsys_run(LinSysSolver* s, OSQPInt iters, OSQPInt eq_rows, 
                                OSQPVectorf* delta_x, OSQPVectorf* z, OSQPVectorf* y, OSQPVectorf* delta_y,
                                const OSQPVectorf* q, const OSQPVectorf* l, const OSQPVectorf* u,
                                const OSQPVectorf* rho_inv);
+/* Builds what osqp_amd_linsys_run needs for a problem with (eq_rows) or
+ * without equality rows, once; the first run does it where this was not
+ * called.  Returns whether the path is on.  Memory that cannot be had leaves
+ * it off and is no error: the caller then iterates as usual. */
+OSQPInt    osqp_amd_linsys_run_prepare(LinSysSolver* s, OSQPInt eq_rows);
 /* Whether the last osqp_amd_linsys_run gave up on the device: its workgroups
  * wait for each other, and a wait that lasts too long (a workgroup that never
  * got onto the GPU) ends the launch.  1: x, z, y and the solver's state are

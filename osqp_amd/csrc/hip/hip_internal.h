@@ -55,6 +55,7 @@ inline int reduce_grid(long long n) {
 }
 
 void* dev_alloc(size_t bytes);           // stream-ordered device allocation
+void* dev_try_alloc(size_t bytes);       // the same; a failure is the caller's to handle and is not recorded
 void dev_free(void* p);
 void upload(void* dst, const void* src, size_t bytes);    // host or device src
 void download(void* dst, const void* src, size_t bytes);  // host or device dst; syncs

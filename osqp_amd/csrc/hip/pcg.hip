@@ -852,6 +852,8 @@ struct HipPcg {
   Runner run;
   RunCall run_call;
   int run_open, run_solves, run_z_count, run_failed;
+  int run_tried;        // builds tried: 1 the one-workgroup kernel, 3 any
+  int run_polls;        // RunCall::polls
   long long run_iters;  // ADMM iterations the runner has done
 };
 
@@ -1114,6 +1116,11 @@ void update_precond(HipPcg* s) {
     hipLaunchKernelGGL(k_recip_to<double>, dim3(grid_for(s->n, kBlock, 4096)), dim3(kBlock), 0, S(), s->n,
                        (const double*)s->dtmp, (double*)s->dinv, none);
   LAUNCHCHK();
+}
+
+void update_precond_if_stale(HipPcg* s) {
+  if (s->kver_P != s->P->version || s->kver_A != s->A->version || (s->bits == 32 && s->A->fp32_dirty))
+    update_precond(s);
 }
 
 // Host-side stop rule: before queueing iteration `it`, look at the flag of
@@ -1512,8 +1519,7 @@ OSQPInt pcg_solve(LinSysSolver* self, OSQPVectorf* b, OSQPInt admm_iter) {
       s->d_flags = nullptr;
     }
   }
-  if (s->kver_P != s->P->version || s->kver_A != s->A->version || (s->bits == 32 && s->A->fp32_dirty))
-    update_precond(s);
+  update_precond_if_stale(s);
   osqp_amd_sec_push(OSQP_AMD_SEC_LINSYS_SOLVE);
   if (s->bits == 32) {
     solve_impl<float>(s, b, admm_iter);
@@ -1673,15 +1679,7 @@ OSQPInt osqp_algebra_init_linsys_solver(LinSysSolver** sp, const OSQPMatrix* P, 
   double cg_bytes = 0.0;
   osqp_amd_linsys_bytes(&s->base, &cg_bytes, nullptr);
   s->lookahead = cg_bytes > 64e6 ? 0 : 2;
-  // The runner multiplies by CG-precision copies throughout: with the FP32 CG
-  // only where the defect correction reads FP32 copies anyway.
-  const bool copies = s->bits == 64 || (s->dcK32 && s->dcA32);
-  if (!polishing && rho_vec && copies && runner_build(&s->run, A, P, RunK{s->krp, s->kci, s->kval64}, s->bits,
-                                                     sizeof(PcgState) / sizeof(double))) {
-    pcg_free(&s->base);
-    *sp = nullptr;
-    return OSQP_LINSYS_SOLVER_INIT_ERROR;
-  }
+  s->run_polls = -1;
   return 0;
 }
 
@@ -1701,17 +1699,41 @@ static bool one_panel(const HipPcg* s) {
          (s->bits == 64 || (one(panels_A<float>(s)) && one(panels_K<float>(s))));
 }
 
+// Builds the runner at the first use that may take it: with equality rows only
+// the one-workgroup kernel (a problem that keeps the separate kernels pays for
+// no copies of A).  Without it, for whatever reason, the separate kernels run.
+OSQPInt osqp_amd_linsys_run_prepare(LinSysSolver* ls, OSQPInt eq_rows) {
+  HipPcg* s = (HipPcg*)ls;
+  if (!s || s->polishing || !s->rho_vec || (eq_rows && !one_panel(s))) return 0;
+  const int tries = eq_rows ? 1 : 3;
+  if (!s->run.on && (s->run_tried | tries) != s->run_tried) {
+    s->run_tried |= tries;
+    update_precond_if_stale(s);
+    // The runner multiplies by CG-precision copies throughout: with the FP32 CG
+    // only where the defect correction reads FP32 copies anyway.
+    if (s->bits == 64 || (s->dcK32 && s->dcA32))
+      runner_build(&s->run, s->A, s->P, RunK{s->krp, s->kci, s->kval64}, s->bits, eq_rows != 0,
+                   sizeof(PcgState) / sizeof(double));
+  }
+  return s->run.on && !(eq_rows && s->run.G > 1);
+}
+
+// the runner off for good (its memory is reused after the work queued so far)
+static void run_off(HipPcg* s) {
+  runner_free(&s->run);
+  s->run_tried = 3;
+  s->run_failed++;
+}
+
 OSQPInt osqp_amd_linsys_run(LinSysSolver* ls, OSQPInt iters, OSQPInt eq_rows, OSQPFloat alpha, OSQPVectorf* x,
                             OSQPVectorf* delta_x, OSQPVectorf* z, OSQPVectorf* y, OSQPVectorf* delta_y,
                             const OSQPVectorf* q, const OSQPVectorf* l, const OSQPVectorf* u,
                             const OSQPVectorf* rho_inv) {
   HipPcg* s = (HipPcg*)ls;
-  if (!s || !s->run.on || iters <= 0 || s->polishing || !s->rho_vec) return 0;
-  if (eq_rows && (s->run.G > 1 || !one_panel(s))) return 0;
-  if (!s->h_flags || s->run_open) return 0;
+  if (!s || iters <= 0 || !s->h_flags || s->run_open) return 0;
   if (!s->ax_valid || s->ax_Aver != s->A->version) return 0;  // the first iteration builds A x64
-  if (s->kver_P != s->P->version || s->kver_A != s->A->version || (s->bits == 32 && s->A->fp32_dirty))
-    update_precond(s);
+  if (!osqp_amd_linsys_run_prepare(ls, eq_rows)) return 0;
+  update_precond_if_stale(s);
   static_assert(sizeof(PcgState) % sizeof(double) == 0, "the state is saved as doubles");
   RunCall c;
   c.iters = iters;
@@ -1740,11 +1762,11 @@ OSQPInt osqp_amd_linsys_run(LinSysSolver* ls, OSQPInt iters, OSQPInt eq_rows, OS
   c.st = RunState{&st->eps_prev, &st->red_factor, &st->zero_iters, &st->iter, &st->solves, &st->active, &st->done,
                   &st->total_iters};
   c.state = (double*)st;
+  c.polls = s->run_polls;
   c.bad = s->d_flags + s->flags_len;
   int z_count = 0;
   if (runner_run(&s->run, s->A, s->P, RunK{s->krp, s->kci, s->kval64}, c, &z_count)) {
-    s->run.on = 0;
-    s->run_failed++;
+    run_off(s);
     return 0;
   }
   s->run_open = s->run.G > 1;
@@ -1771,8 +1793,7 @@ OSQPInt osqp_amd_linsys_run_failed(LinSysSolver* ls, OSQPInt waited) {
   s->host_solves = s->run_solves;
   s->z_count = s->run_z_count;
   s->run_iters -= s->run_call.iters;
-  s->run.on = 0;
-  s->run_failed++;
+  run_off(s);
   return 1;
 }
 
@@ -1787,7 +1808,7 @@ OSQPInt osqp_amd_linsys_run_stats(LinSysSolver* ls, long long* iters, OSQPInt* g
 
 void osqp_amd_linsys_run_polls(LinSysSolver* ls, OSQPInt polls) {
   HipPcg* s = (HipPcg*)ls;
-  if (s && polls >= 0) s->run.polls = polls;
+  if (s && polls >= 0) s->run_polls = polls;
 }
 
 // Times the two CG operator kernels (w = rho o A p and Kp = sigma p + P p + A' w)

@@ -68,7 +68,6 @@ struct Runner {
   double* xch;        // 2 n: r64, K p
   unsigned* bar;      // barrier words
   double* save;       // what a launch changes, as it was before it (runner_restore)
-  int polls;          // a barrier's wait gives up after this many looks
   long long ver_A, ver_P;  // versions the values were copied from
 };
 
@@ -94,13 +93,15 @@ struct RunCall {
   const void* dinv;                                 // CG precision
   RunState st;
   double* state;                                    // the PCG's device state (Runner::state_len)
-  int* bad;           // host-coherent word, set where a barrier gave up
+  int polls;          // looks after which a barrier's wait gives up (-1: the default)
+  int* bad;           // host-coherent word, set where that happened
 };
 
-// Builds the runner for A (m x n, CSR and CSC on the device) when it pays and
-// fits; r->on stays 0 otherwise.  Returns 1 on an allocation failure.
-// state_len: doubles of the PCG's device state.
-int runner_build(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P, const RunK& k, int bits, int state_len);
+// Builds the runner for A (m x n, CSR and CSC on the device) when it pays, fits
+// and its memory can be had; r->on stays 0 and r empty otherwise.  Returns
+// r->on.  one: only the one-workgroup kernel will do.  state_len: doubles of
+// the PCG's device state.
+int runner_build(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P, const RunK& k, int bits, bool one, int state_len);
 void runner_free(Runner* r);
 // Queues c.iters ADMM iterations and leaves the new z_count; 1 when the launch
 // was refused (nothing has changed then).

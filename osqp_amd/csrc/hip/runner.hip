@@ -4,6 +4,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <new>
 #include <vector>
 
 #include "panel.h"
@@ -1156,9 +1157,9 @@ int build_op(Runner* r, RunOp* o, const OSQPMatrix* M, int* d_steps, int* h_step
   const int per = kWave >> o->lgT;
   o->ns = (rows + per - 1) / per;
   if (o->ns < 1) o->ns = 1;
-  o->soff = (int*)dev_alloc(sizeof(int) * (size_t)G * (o->ns + 1));
-  o->perm = (uint16_t*)dev_alloc(sizeof(uint16_t) * (size_t)G * o->ns * per);
-  o->base = (long long*)dev_alloc(sizeof(long long) * (G + 1));
+  o->soff = (int*)dev_try_alloc(sizeof(int) * (size_t)G * (o->ns + 1));
+  o->perm = (uint16_t*)dev_try_alloc(sizeof(uint16_t) * (size_t)G * o->ns * per);
+  o->base = (long long*)dev_try_alloc(sizeof(long long) * (G + 1));
   if (!o->soff || !o->perm || !o->base) return 1;
   int N = 1;
   while (N < rows) N <<= 1;
@@ -1180,8 +1181,8 @@ int build_op(Runner* r, RunOp* o, const OSQPMatrix* M, int* d_steps, int* h_step
 
 int alloc_op(Runner* r, RunOp* o) {
   const size_t e = (size_t)(o->steps > 0 ? o->steps : 1) * kWave;
-  o->col = (uint16_t*)dev_alloc(sizeof(uint16_t) * e);
-  o->val = dev_alloc((size_t)(r->bits / 8) * e);
+  o->col = (uint16_t*)dev_try_alloc(sizeof(uint16_t) * e);
+  o->val = dev_try_alloc((size_t)(r->bits / 8) * e);
   return !o->col || !o->val;
 }
 
@@ -1261,8 +1262,8 @@ int build_op1(RunOp* o, const std::vector<int>& rp, int bits) {  // bits: of the
   o->slots = (int)perm.size();
   sl.push_back(make_int2(at, 0));
   o->steps = o->max_steps = at;
-  o->soff = (int*)dev_alloc(sizeof(int2) * sl.size());
-  o->perm = (uint16_t*)dev_alloc(sizeof(uint16_t) * (perm.empty() ? 1 : perm.size()));
+  o->soff = (int*)dev_try_alloc(sizeof(int2) * sl.size());
+  o->perm = (uint16_t*)dev_try_alloc(sizeof(uint16_t) * (perm.empty() ? 1 : perm.size()));
   if (!o->soff || !o->perm) return 1;
   upload(o->soff, sl.data(), sizeof(int2) * sl.size());
   upload(o->perm, perm.data(), sizeof(uint16_t) * perm.size());
@@ -1337,11 +1338,14 @@ void runner_free(Runner* r) {
 static int build_many(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P) {
   const int n = r->n, G = r->G;
   r->cw = (n + G - 1) / G;
-  r->r0 = (int*)dev_alloc(sizeof(int) * (G + 2));
-  r->cs = (int*)dev_alloc(sizeof(int) * (size_t)(G + 1) * n);
-  int* d_steps = (int*)dev_alloc(sizeof(int) * G);
+  r->r0 = (int*)dev_try_alloc(sizeof(int) * (G + 2));
+  r->cs = (int*)dev_try_alloc(sizeof(int) * (size_t)(G + 1) * n);
+  struct Steps {
+    int* p;
+    ~Steps() { dev_free(p); }
+  } d_steps{(int*)dev_try_alloc(sizeof(int) * G)};
   std::vector<int> h((size_t)G + 2);
-  int rc = !r->r0 || !r->cs || !d_steps;
+  int rc = !r->r0 || !r->cs || !d_steps.p;
   bool fits = !rc;
   if (!rc) {
     const int one = 1;
@@ -1357,20 +1361,19 @@ static int build_many(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P) {
     fits = h[(size_t)G + 1] == 1 && r->rows_max < kSortMax && r->lds <= kRunLds;
   }
   if (fits) {
-    rc = build_op<kRowsA>(r, &r->A, A, d_steps, h.data()) || build_op<kColsA>(r, &r->At, A, d_steps, h.data()) ||
-         build_op<kRowsP>(r, &r->P, P, d_steps, h.data());
+    rc = build_op<kRowsA>(r, &r->A, A, d_steps.p, h.data()) || build_op<kColsA>(r, &r->At, A, d_steps.p, h.data()) ||
+         build_op<kRowsP>(r, &r->P, P, d_steps.p, h.data());
     for (const RunOp* o : {&r->A, &r->At, &r->P}) r->lds = ((r->lds + 15) & ~(size_t)15) + run_lds_list(o->lgT, o->ns) + 16;
     fits = !rc && op_fits(r, r->A, A->nnz) && op_fits(r, r->At, A->nnz) && op_fits(r, r->P, P->nnz) && r->lds <= kRunLds;
   }
-  dev_free(d_steps);
   if (rc || !fits) {
     r->G = 0;
     return rc;
   }
-  r->part = (double*)dev_alloc(sizeof(double) * (size_t)G * n);
-  r->xch = (double*)dev_alloc(sizeof(double) * 2 * (size_t)n);
-  r->bar = (unsigned*)dev_alloc(sizeof(unsigned) * kBarWords);
-  r->save = (double*)dev_alloc(sizeof(double) * run_save_len(n, r->m, r->state_len));
+  r->part = (double*)dev_try_alloc(sizeof(double) * (size_t)G * n);
+  r->xch = (double*)dev_try_alloc(sizeof(double) * 2 * (size_t)n);
+  r->bar = (unsigned*)dev_try_alloc(sizeof(unsigned) * kBarWords);
+  r->save = (double*)dev_try_alloc(sizeof(double) * run_save_len(n, r->m, r->state_len));
   if (alloc_op(r, &r->A) || alloc_op(r, &r->At) || alloc_op(r, &r->P) || !r->part || !r->xch || !r->bar || !r->save) return 1;
   fill_A(r, A, true);
   fill_P(r, P, true);
@@ -1382,8 +1385,7 @@ static int build_many(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P) {
   return 0;
 }
 
-int runner_build(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P, const RunK& k, int bits, int state_len) {
-  memset(r, 0, sizeof(*r));
+static int build_any(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P, const RunK& k, int bits, bool one, int state_len) {
   const int n = A->n, m = A->m;
   if (A->is_triu || n <= 0 || m <= 0 || A->nnz <= 0 || n > run_n_max(bits)) return 0;
   const long long work = (long long)A->nnz + P->nnz;
@@ -1397,7 +1399,7 @@ int runner_build(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P, const RunK
     rc = build1(r, A, P, k);
     if (rc || r->G == 0) runner_free(r);
   }
-  if (!rc && r->G == 0) {
+  if (!rc && r->G == 0 && !one) {
     // Measured us per ADMM iteration with G = 32 / 64 / 128 / 256 workgroups:
     // 108k entries 33 / - / - / -, 180k 39 / 36 / 37 / 39, 624k 52 / 48 / 43 /
     // 46, 1.4M 62 / 50 / 46 / 48 (FP64): a workgroup's share against the
@@ -1409,19 +1411,24 @@ int runner_build(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P, const RunK
     r->bits = bits;
     r->G = G;
     r->state_len = state_len;
-    r->polls = kRunPolls;
     rc = build_many(r, A, P);
   }
-  if (rc || r->G == 0) {
-    runner_free(r);
-    return rc;
-  }
-  if (HIPCHK(hipFuncSetAttribute(kernel_of(r), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kRunLds))) {
-    runner_free(r);
+  if (rc || r->G == 0) return 0;
+  if (hipFuncSetAttribute(kernel_of(r), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kRunLds) != hipSuccess) {
+    (void)hipGetLastError();
     return 0;
   }
-  r->on = LAUNCHCHK() == 0;
-  return 0;
+  return LAUNCHCHK() == 0;
+}
+
+int runner_build(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P, const RunK& k, int bits, bool one, int state_len) {
+  memset(r, 0, sizeof(*r));
+  try {
+    r->on = build_any(r, A, P, k, bits, one, state_len);
+  } catch (const std::bad_alloc&) {
+  }
+  if (!r->on) runner_free(r);
+  return r->on;
 }
 
 static void run_save(const Runner* r, const RunCall& c, int back) {
@@ -1456,7 +1463,7 @@ int runner_run(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P, const RunK& 
   a.part = r->part;
   a.xch = r->xch;
   a.bar = r->bar;
-  a.polls = r->polls;
+  a.polls = c.polls >= 0 ? c.polls : kRunPolls;
   a.c = c;
   void* args[] = {&a};
   hipError_t err;

@@ -45,7 +45,7 @@ static size_t bucket_of(size_t bytes) {
   return b;
 }
 
-void* dev_alloc(size_t bytes) {
+static void* alloc_block(size_t bytes, bool record) {
   if (bytes == 0) bytes = 1;
   size_t b = bucket_of(bytes);
   std::lock_guard<std::mutex> lk(g_mu);
@@ -68,11 +68,18 @@ void* dev_alloc(size_t bytes) {
     g_cache.free_lists.clear();
     g_cache.cached_bytes = 0;
     (void)hipGetLastError();
-    if (HIPCHK(hipMalloc(&p, b))) return nullptr;
+    const hipError_t e = hipMalloc(&p, b);
+    if (e != hipSuccess) {
+      if (record) HIPCHK(e);
+      else (void)hipGetLastError();
+      return nullptr;
+    }
   }
   g_cache.sizes[p] = b;
   return p;
 }
+void* dev_alloc(size_t bytes) { return alloc_block(bytes, true); }
+void* dev_try_alloc(size_t bytes) { return alloc_block(bytes, false); }
 
 // Blocks go back to the cache; reuse is ordered after earlier work because all
 // kernels and copies run on the single backend stream.

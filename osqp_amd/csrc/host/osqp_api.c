@@ -114,6 +114,24 @@ static OSQPSettings* copy_settings(const OSQPSettings* s) {
   return c;
 }
 
+/* ADMM iterations from `iter` on that the loop of osqp_solve runs without
+ * looking at them on the host: up to the next termination check, rho update,
+ * printed line or the last iteration.  0 where it looks at every one: the
+ * first iteration, a time limit, section markers, a rho interval not yet
+ * fixed, scalar rho. */
+static OSQPInt free_iterations(const OSQPSolver* solver, OSQPInt iter) {
+  const OSQPSettings* s = solver->settings;
+  OSQPInt k = s->max_iter - iter + 1, every[3], j;
+  if (iter == 1 || !s->rho_is_vec || s->profiler_level || s->time_limit < OSQP_TIME_LIMIT) return 0;
+  if (s->adaptive_rho != OSQP_ADAPTIVE_RHO_UPDATE_DISABLED && s->adaptive_rho_interval == 0) return 0;
+  every[0] = s->check_termination;
+  every[1] = s->adaptive_rho != OSQP_ADAPTIVE_RHO_UPDATE_DISABLED ? s->adaptive_rho_interval : 0;
+  every[2] = s->verbose ? OSQP_PRINT_INTERVAL : 0;
+  for (j = 0; j < 3; j++)
+    if (every[j] > 0) k = c_min(k, every[j] - (iter - 1) % every[j]);
+  return c_min(k, 64);  /* an interrupt is seen between launches */
+}
+
 /* ---- setup: src/osqp_api.c:332-631 ------------------------------------------ */
 #define ALLOC_OR_FAIL(ptr) do { if (!(ptr)) return osqp_error(OSQP_MEM_ALLOC_ERROR); } while (0)
 
@@ -328,6 +346,7 @@ static OSQPInt setup_workspace(OSQPSolver** solverp, const OSQPCscMatrix* P, con
   } else if (exitflag) {
     return osqp_error(exitflag);
   }
+  if (free_iterations(solver, 2) > 0) osqp_amd_linsys_run_prepare(work->linsys_solver, work->eq_rows);
 
   osqp_cold_start(solver);
 
@@ -392,24 +411,6 @@ static void print_summary(const OSQPSolver* solver) {
   printf("%4d  % 12.4e  %9.2e  %9.2e  %9.2e  %.1es\n", (int)info->iter, info->obj_val, info->prim_res,
          info->dual_res, solver->settings->rho, info->solve_time);
   solver->work->summary_printed = 1;
-}
-
-/* ADMM iterations from `iter` on that the loop of osqp_solve runs without
- * looking at them on the host: up to the next termination check, rho update,
- * printed line or the last iteration.  0 where it looks at every one: the
- * first iteration, a time limit, section markers, a rho interval not yet
- * fixed, scalar rho. */
-static OSQPInt free_iterations(const OSQPSolver* solver, OSQPInt iter) {
-  const OSQPSettings* s = solver->settings;
-  OSQPInt k = s->max_iter - iter + 1, every[3], j;
-  if (iter == 1 || !s->rho_is_vec || s->profiler_level || s->time_limit < OSQP_TIME_LIMIT) return 0;
-  if (s->adaptive_rho != OSQP_ADAPTIVE_RHO_UPDATE_DISABLED && s->adaptive_rho_interval == 0) return 0;
-  every[0] = s->check_termination;
-  every[1] = s->adaptive_rho != OSQP_ADAPTIVE_RHO_UPDATE_DISABLED ? s->adaptive_rho_interval : 0;
-  every[2] = s->verbose ? OSQP_PRINT_INTERVAL : 0;
-  for (j = 0; j < 3; j++)
-    if (every[j] > 0) k = c_min(k, every[j] - (iter - 1) % every[j]);
-  return c_min(k, 64);  /* an interrupt is seen between launches */
 }
 
 /* ---- solve: src/osqp_api.c:636-1038 ---------------------------------------- */

@@ -189,3 +189,32 @@ def test_equality_rows_keep_the_separate_kernels_order(features, precision):
     assert a[1][3] == b[1][3] == 1
     c = pr.kkt_certificate(dict(p, **relaxed), b[1][0], b[1][1])
     assert c["prim"] <= 1e-4 + 1e-4 * c["scale_p"] and c["dual"] <= 1e-4 + 1e-4 * c["scale_d"]
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+def test_built_where_it_can_run(precision):
+    """With equality rows the several-workgroup kernel is not built; it is once they are gone, and a solver
+    that never iterates many at a time builds none."""
+    p = qp(700, 9001, 30, seed=2)
+    ax = p["A"] @ np.random.default_rng(3).uniform(-0.01, 0.01, 700)
+    l, u = p["l"].copy(), p["u"].copy()
+    l[:5] = u[:5] = ax[:5]
+    s = OSQP(precision=precision)
+    assert s.setup(p["P"], p["q"], p["A"], l, u, **EPS) == 0
+    assert s.run_stats().groups == 0
+    s.solve()
+    assert (s.run_stats().groups, s.run_stats().iters) == (0, 0)
+    s.update(l=p["l"], u=p["u"])
+    r = s.solve()
+    assert s.run_stats().groups > 1 and s.run_stats().iters == r.info.iter - 1
+    s.update(l=l, u=u)  # equality rows again: built, not used
+    s.solve()
+    assert s.run_stats().iters == r.info.iter - 1
+    s.close()
+    q = qp(300, 3000, 20, seed=2)
+    for st, groups in ((dict(), True), (dict(time_limit=100.0), False), (dict(profiler_level=1), False)):
+        s = OSQP(precision=precision)
+        assert s.setup(q["P"], q["q"], q["A"], q["l"], q["u"], **EPS, **st) == 0
+        s.solve()
+        assert (s.run_stats().groups > 1, s.run_stats().iters > 0) == (groups, groups)
+        s.close()
