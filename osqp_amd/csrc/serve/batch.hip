@@ -359,8 +359,19 @@ constexpr int kSlicedBucket = 3;
 // 512 MPC problems of horizons 10..50 from 60.0 to 31.9 ms (FP32), 24 of them
 // from 18.6 to 10.7 ms (FP64), 12 resident portfolios of 500..1000 assets from
 // 621 to 300 ms, the same bits.  A row in between has more pieces than the
-// left-to-right sum keeps in the group walk's order.
+// left-to-right sum keeps in the group walk's order.  Up to kLaneCols columns
+// the ADMM step laid out for lane rows takes them (Solver::lane_admm, FP64: one
+// reduction block a wavefront); past that only FP32, and only rows that the
+// lanes do not pad too much: permuted problems (n = m) of 3, 6, 10 entries a
+// row, time on the row groups over time on lane rows, 1 / 16 / 256 problems in
+// flight: n = 2000 FP32 1.43 / 1.42 / 1.22, 1.36 / 1.34 / 1.07, 1.61 / 1.57 /
+// 1.17, FP64 1.27 / 1.38 / 1.20, 1.10 / 1.16 / 1.02, 1.37 / 1.40 / 1.11;
+// n = 3000 FP32 1.17 / 1.15 / 0.96, 1.30 / 1.31 / 1.05, 1.58 / 1.58 / 1.22,
+// FP64 0.63 / 0.88 / 0.74, 0.93 / 0.85 / 0.90, 0.91 / 0.97 / 0.97.  Slots over
+// entries there: 5.4, 3.2, 2.0.
 constexpr int kLaneBuckets = 3;
+constexpr int kLaneCols = kMaxTeamWaves * kRedBlock;
+constexpr double kLanePad = 4.5;
 
 // medium rows in slice order: longest first, row order among equals
 void ell_order(const int* rp, int rows, std::vector<int>* order) {
@@ -734,6 +745,12 @@ Layout build_host(HostData* h, int vbytes, const OSQPCscMatrix* P, const OSQPFlo
     h->gP.lane_slots = lane_layout(prp.data(), n, nullptr, nullptr);
     h->gA.lane_slots = lane_layout(arp.data(), m, nullptr, nullptr);
     h->gT.lane_slots = lane_layout(A->p, n, nullptr, nullptr);
+    const double slots = (double)(h->gP.lane_slots + h->gA.lane_slots + h->gT.lane_slots);
+    if (n > kLaneCols && (vbytes == 8 || slots > kLanePad * (double)(h->nnzP + 2LL * h->nnzA)))
+      for (GroupDims* g : {&h->gP, &h->gA, &h->gT}) {
+        g->lanes = false;
+        g->lane_slots = 0;
+      }
   }
   h->warm_x = x0 != nullptr;
   h->warm_y = y0 != nullptr;

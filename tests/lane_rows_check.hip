@@ -126,9 +126,10 @@ int main(int argc, char** argv) {
     for (int vbytes : {4, 8}) {
       HostData h;
       const Layout L = build_host(&h, vbytes, &M[0], q.data(), &M[1], l.data(), u.data(), nullptr, nullptr, false);
-      CHECK(h.gA.lanes == (want != 0) && h.gP.lanes == h.gA.lanes && h.gT.lanes == h.gA.lanes, "problem %d: lane rows %d", t,
+      const bool lane = want == 1 || (want == 2 && vbytes == 4);  // 2: in FP32 alone
+      CHECK(h.gA.lanes == lane && h.gP.lanes == h.gA.lanes && h.gT.lanes == h.gA.lanes, "problem %d: lane rows %d", t,
             (int)h.gA.lanes);
-      CHECK(bucket_of(h) == (want ? kBuckets : 0) + size_bucket(n, m, h.nnzA, h.nnzP), "problem %d: bucket", t);
+      CHECK(bucket_of(h) == (lane ? kBuckets : 0) + size_bucket(n, m, h.nnzA, h.nnzP), "problem %d: bucket", t);
       if (!h.gA.lanes) continue;
       lanes++;
       std::vector<char> blk(L.total + 64, 0);

@@ -26,6 +26,15 @@ def _short_rows(m, n, lens, seed):
     return dict(P=sp.diags(1.0 + rng.random(n), format="csc"), A=sp.csc_matrix(A))
 
 
+def _circulant(n, per):
+    """A with entry (r, (r + k) mod n) for k < per: rows and columns of `per` entries; P a band of the same."""
+    rng = np.random.default_rng(n + per)
+    r = np.repeat(np.arange(n), per)
+    A = sp.csc_matrix((rng.standard_normal(n * per), (r, (r + np.tile(np.arange(per), n)) % n)), shape=(n, n))
+    return dict(P=sp.diags([1.0 + rng.random(n - k) for k in range((per + 1) // 2)], list(range((per + 1) // 2)),
+                           format="csc"), A=A)
+
+
 def _problems():
     out = [(pr.mpc(N, seed=N), 1) for N in (1, 10, 33, 50)]
     out.append((_short_rows(1, 1, [1], 1), 1))
@@ -37,6 +46,9 @@ def _problems():
     p = _short_rows(100, 100, [3], 6)
     p["A"] = sp.vstack([p["A"], sp.csc_matrix((1, 100))], format="csc")
     out.append((p, 0))                                  # an empty row
+    # past 2048 columns: FP32 alone, and rows that the lanes do not pad too much
+    out += [(_circulant(2048, 9), 1), (_circulant(2049, 9), 2), (_circulant(4096, 5), 2), (_circulant(4097, 5), 0),
+            (_circulant(2048, 3), 1), (_circulant(2049, 3), 0)]
     return out
 
 
