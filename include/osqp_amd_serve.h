@@ -68,7 +68,10 @@ typedef struct {
 
 /* precision: 32 (FP32 CG, FP64 residuals and ADMM state) or 64.
  * max_active: problems on the GPU at once (0: 4096).
- * arena_bytes: device memory for resident problems (0: 4 GiB).
+ * arena_bytes: device memory for resident problems (0: 4 GiB; 1/64 more is
+ * allocated for row tables).  The first small problem of short rows allocates
+ * as much again, at most 4 GiB, for copies that its kernel reads faster; a
+ * problem that finds no room there runs without, with the same results.
  * Pinned host memory: a staging pool of arena_bytes / 4 (at least 64 MiB, at
  * most 1 GiB) for stage images, results and matrix updates, and an image arena
  * of half the pool's size where osqp_batch_add builds stage images (when it
@@ -175,6 +178,10 @@ OSQPInt osqp_batch_set_team(OSQPBatch* batch, OSQPInt bucket, OSQPInt team, OSQP
 /* Engine counters: epochs run, ADMM iterations, GPU time of the epochs (s:
  * the time during which at least one bucket's epoch ran). */
 OSQPInt osqp_batch_counters(const OSQPBatch* batch, long long* epochs, long long* admm_iters, OSQPFloat* gpu_s);
+
+/* Problems admitted so far, and those of them on lane rows (the kernel for
+ * small problems of short rows).  Returns 0 or -1. */
+OSQPInt osqp_batch_lanes(const OSQPBatch* batch, long long* admitted, long long* on_lanes);
 
 OSQPInt osqp_batch_destroy(OSQPBatch* batch);
 

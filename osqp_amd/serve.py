@@ -70,6 +70,8 @@ def _bind(lib):
     lib.osqp_batch_counters.argtypes = [vp, C.POINTER(C.c_longlong), C.POINTER(C.c_longlong),
                                         C.POINTER(C.c_double)]
     lib.osqp_batch_counters.restype = C.c_int
+    lib.osqp_batch_lanes.argtypes = [vp, C.POINTER(C.c_longlong), C.POINTER(C.c_longlong)]
+    lib.osqp_batch_lanes.restype = C.c_int
     lib.osqp_batch_destroy.argtypes = [vp]
     lib.osqp_batch_destroy.restype = C.c_int
     _bound = True
@@ -259,6 +261,12 @@ class BatchEngine:
         e, i, g = C.c_longlong(0), C.c_longlong(0), C.c_double(0)
         self.lib.osqp_batch_counters(self._b, C.byref(e), C.byref(i), C.byref(g))
         return dict(epochs=e.value, admm_iters=i.value, gpu_s=g.value)
+
+    def lanes(self):
+        """(problems admitted so far, those of them on lane rows)."""
+        a, k = C.c_longlong(0), C.c_longlong(0)
+        self.lib.osqp_batch_lanes(self._b, C.byref(a), C.byref(k))
+        return a.value, k.value
 
     # ---- convenience ----------------------------------------------------------
     def solve_batch(self, problems, max_epochs=100000):

@@ -42,7 +42,7 @@ static void check(const char* name, const char* blk, size_t total, int rows, int
   const unsigned char* lc0 = (const unsigned char*)(blk + o.lc0);
   const int nls = lane_slices(rows);
   CHECK(nls <= kWave, "%s: slices", name);
-  CHECK(o.lcol + 2 * (size_t)d.lane_slots <= total && o.lrv64 + 8 * (size_t)d.lane_slots <= total, "%s: block", name);
+  CHECK(o.lcol + 2 * (size_t)d.lane_slots <= total && o.lrv64 + 8 * (size_t)d.lane_slots <= total, "%s: lane block", name);
   std::vector<int> col((size_t)d.lane_slots, -1);
   std::vector<double> v((size_t)d.lane_slots, -1.0);
   for (int w = 0; w < nls * kWave; ++w) {
@@ -144,9 +144,9 @@ int main(int argc, char** argv) {
       for (int pass = 0; pass < 2; ++pass) {
         auto one = [&](auto zero) {
           using T = decltype(zero);
-          check<T>("P", blk.data(), L.total, n, n, h.gP, L.gP, L.Prp, L.Pci, L.Pval);
-          check<T>("A", blk.data(), L.total, m, n, h.gA, L.gA, L.Arp, L.Aci, L.Aval);
-          check<T>("At", blk.data(), L.total, n, m, h.gT, L.gT, L.Trp, L.Tci, L.Tval);
+          check<T>("P", blk.data(), L.lane_total, n, n, h.gP, L.gP, L.Prp, L.Pci, L.Pval);
+          check<T>("A", blk.data(), L.lane_total, m, n, h.gA, L.gA, L.Arp, L.Aci, L.Aval);
+          check<T>("At", blk.data(), L.lane_total, n, m, h.gT, L.gT, L.Trp, L.Tci, L.Tval);
         };
         if (pass == 0) one(0.0);
         else one(0.0f);
