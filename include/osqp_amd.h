@@ -284,10 +284,12 @@ OSQPInt osqp_amd_solver_stats(OSQPSolver* solver, OSQPInt* pcg_iters_total,
                               OSQPInt* linsys_solves, double* gpu_ms);
 
 /* The ADMM iterations that this solver has run many to a launch, the launch's
- * workgroups (0: that path is off) and the launches that gave up or were
- * refused, whose iterations the separate kernels did (any may be null; see
- * osqp_amd_linsys_run in osqp_amd_algebra.h). */
-OSQPInt osqp_amd_solver_run_stats(OSQPSolver* solver, long long* iters, OSQPInt* groups, OSQPInt* failed);
+ * workgroups (0: that path is off), the entries of a row that one lane adds up
+ * at most and the launches that gave up or were refused, whose iterations the
+ * separate kernels did (any may be null; see osqp_amd_linsys_run in
+ * osqp_amd_algebra.h). */
+OSQPInt osqp_amd_solver_run_stats(OSQPSolver* solver, long long* iters, OSQPInt* groups, OSQPInt* chain,
+                                  OSQPInt* failed);
 /* Looks after which a wait between such a launch's workgroups gives up (for
  * checks; the default is some seconds' worth).  Returns 0, or 1 when polls < 0
  * or the solver has none. */

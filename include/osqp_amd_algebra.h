@@ -232,8 +232,10 @@ OSQPInt    osqp_amd_linsys_run_prepare(LinSysSolver* s, OSQPInt eq_rows);
  * received a result queued after the run, so there is nothing to wait for. */
 OSQPInt    osqp_amd_linsys_run_failed(LinSysSolver* s, OSQPInt waited);
 /* ADMM iterations done by osqp_amd_linsys_run, its workgroups (0: the path is
- * off) and the runs that gave up or were refused. */
-OSQPInt    osqp_amd_linsys_run_stats(LinSysSolver* s, long long* iters, OSQPInt* groups, OSQPInt* failed);
+ * off), the entries of a row that one lane adds up at most (several
+ * workgroups) and the runs that gave up or were refused. */
+OSQPInt    osqp_amd_linsys_run_stats(LinSysSolver* s, long long* iters, OSQPInt* groups, OSQPInt* chain,
+                                     OSQPInt* failed);
 /* Looks after which a workgroup's wait gives up, for this solver (checks). */
 void       osqp_amd_linsys_run_polls(LinSysSolver* s, OSQPInt polls);
 /* Queued reductions (no counterpart in the reference, whose reductions each

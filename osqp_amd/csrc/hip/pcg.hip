@@ -1797,11 +1797,13 @@ OSQPInt osqp_amd_linsys_run_failed(LinSysSolver* ls, OSQPInt waited) {
   return 1;
 }
 
-OSQPInt osqp_amd_linsys_run_stats(LinSysSolver* ls, long long* iters, OSQPInt* groups, OSQPInt* failed) {
+OSQPInt osqp_amd_linsys_run_stats(LinSysSolver* ls, long long* iters, OSQPInt* groups, OSQPInt* chain,
+                                  OSQPInt* failed) {
   HipPcg* s = (HipPcg*)ls;
   if (!s) return 1;
   if (iters) *iters = s->run_iters;
   if (groups) *groups = s->run.on ? s->run.G : 0;
+  if (chain) *chain = s->run.chain;
   if (failed) *failed = s->run_failed;
   return 0;
 }

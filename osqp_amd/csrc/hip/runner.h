@@ -57,6 +57,7 @@ struct Runner {
   int cw;             // columns per chunk
   int rows_max;       // rows of the largest workgroup range
   int resident;       // the copies held in LDS
+  int chain;          // entries that one lane adds up, at most (several workgroups)
   size_t lds;         // dynamic LDS of a launch
   int* r0;            // G + 1 row ranges
   int* cs;            // (G + 1) * n: first entry of column j at or below row r0[b] (CSC positions)

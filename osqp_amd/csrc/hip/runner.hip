@@ -21,6 +21,7 @@ constexpr int kRunRefresh = 8;      // ADMM iterations between two exact recompu
 constexpr uint16_t kNoRow = 0xFFFF;
 constexpr size_t kRunLds = 159 * 1024;  // dynamic LDS of a launch
 constexpr long long kRun1Work = 48000;  // entries of A and P up to which one workgroup runs alone
+constexpr int kRunChain = 24;  // entries that a lane adds up of a row, while a row has lanes left to take
 constexpr int kRunPolls = 1 << 22;  // looks of a barrier's wait, some seconds
 
 inline hipStream_t S() { return rt().stream; }
@@ -131,6 +132,7 @@ __global__ __launch_bounds__(kT) void k_run_layout(RunSrc src, int lgT, int ns, 
     }
     soff[(long long)b * (ns + 1) + ns] = at;
     steps[b] = at;
+    steps[gridDim.x + b] = rows > 0 ? 65535 - (int)(key[0] >> 16) : 0;  // the longest row's
   }
 }
 
@@ -1135,7 +1137,7 @@ void free_op(RunOp* o) {
 }
 
 // lanes per row: enough to give every lane of the workgroup a row share, at
-// most half an average row's entries
+// most half an average row's entries; more where build_op finds a longer chain
 int pick_lgT(long long rows, double len) {
   int lg = 0;
   while (lg < 6 && (rows << lg) < kT && (2 << lg) <= len / 2) ++lg;
@@ -1148,33 +1150,58 @@ RunSrc run_src(const Runner* r, const OSQPMatrix* M) {
                 r->r0, r->cs};
 }
 
-// slices of one copy; 1 on an allocation failure
+// padding at most as much as the entries, and no workgroup far above its share
+bool op_fits(const Runner* r, const RunOp& o, long long nnz) {
+  return o.steps * kWave <= 2 * nnz + 4096LL * r->G && o.max_steps <= 64 + 4 * (nnz / kWave / r->G + 1);
+}
+
+// slices of one copy; 1 on an allocation failure, 2 when it does not fit.  Each lane adds up a chain of
+// its row's entries, then the lanes are added by a tree.  In a panel task of
+// rows of one length, up to 64 lanes' worth, a chain is at most 24 entries long
+// in FP32; so that the error of a sum is no larger here, a copy takes more lanes
+// a row than pick_lgT's until no row's chain is longer than that (a copy that
+// does not fit on pick_lgT's lanes is not taken on more).
 template <RunKind K>
 int build_op(Runner* r, RunOp* o, const OSQPMatrix* M, int* d_steps, int* h_steps) {
   const int rows = K == kColsA ? r->n : K == kRowsA ? r->rows_max : r->cw, G = r->G;
   o->slots = 0;
   o->lgT = pick_lgT(rows, (double)M->nnz / ((double)G * (rows > 0 ? rows : 1)));
-  const int per = kWave >> o->lgT;
-  o->ns = (rows + per - 1) / per;
-  if (o->ns < 1) o->ns = 1;
-  o->soff = (int*)dev_try_alloc(sizeof(int) * (size_t)G * (o->ns + 1));
-  o->perm = (uint16_t*)dev_try_alloc(sizeof(uint16_t) * (size_t)G * o->ns * per);
-  o->base = (long long*)dev_try_alloc(sizeof(long long) * (G + 1));
-  if (!o->soff || !o->perm || !o->base) return 1;
   int N = 1;
   while (N < rows) N <<= 1;
   const size_t kb = sizeof(unsigned) * (size_t)N;
   if (kb > 48 * 1024)
     HIPCHK(hipFuncSetAttribute((const void*)k_run_layout<K>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kb));
-  hipLaunchKernelGGL((k_run_layout<K>), dim3(G), dim3(kT), kb, S(), run_src<K>(r, M), o->lgT, o->ns, o->soff, o->perm,
-                     d_steps);
-  download(h_steps, d_steps, sizeof(int) * G);
-  std::vector<long long> base((size_t)G + 1, 0);
-  for (int b = 0; b < G; ++b) {
-    base[(size_t)b + 1] = base[(size_t)b] + h_steps[b];
-    if (h_steps[b] > o->max_steps) o->max_steps = h_steps[b];
+  o->base = (long long*)dev_try_alloc(sizeof(long long) * (G + 1));
+  if (!o->base) return 1;
+  for (;; ++o->lgT) {
+    const int per = kWave >> o->lgT;
+    o->ns = (rows + per - 1) / per;
+    if (o->ns < 1) o->ns = 1;
+    o->soff = (int*)dev_try_alloc(sizeof(int) * (size_t)G * (o->ns + 1));
+    o->perm = (uint16_t*)dev_try_alloc(sizeof(uint16_t) * (size_t)G * o->ns * per);
+    if (!o->soff || !o->perm) return 1;
+    hipLaunchKernelGGL((k_run_layout<K>), dim3(G), dim3(kT), kb, S(), run_src<K>(r, M), o->lgT, o->ns, o->soff, o->perm,
+                       d_steps);
+    download(h_steps, d_steps, sizeof(int) * 2 * G);
+    int chain = 0;
+    o->steps = o->max_steps = 0;
+    for (int b = 0; b < G; ++b) {
+      chain = std::max(chain, h_steps[G + b]);
+      o->steps += h_steps[b];
+      o->max_steps = std::max(o->max_steps, h_steps[b]);
+    }
+    if (!op_fits(r, *o, M->nnz)) return 2;
+    if (chain <= kRunChain || o->lgT == 6) {
+      r->chain = std::max(r->chain, chain);
+      break;
+    }
+    dev_free(o->soff);
+    dev_free(o->perm);
+    o->soff = nullptr;
+    o->perm = nullptr;
   }
-  o->steps = base[(size_t)G];
+  std::vector<long long> base((size_t)G + 1, 0);
+  for (int b = 0; b < G; ++b) base[(size_t)b + 1] = base[(size_t)b] + h_steps[b];
   upload(o->base, base.data(), sizeof(long long) * base.size());
   return 0;
 }
@@ -1204,11 +1231,6 @@ void fill_A(Runner* r, const OSQPMatrix* A, bool cols) {
 void fill_P(Runner* r, const OSQPMatrix* P, bool cols) {
   fill_op<kRowsP>(r, &r->P, P, cols);
   r->ver_P = P->version;
-}
-
-// padding at most as much as the entries, and no workgroup far above its share
-bool op_fits(const Runner* r, const RunOp& o, long long nnz) {
-  return o.steps * kWave <= 2 * nnz + 4096LL * r->G && o.max_steps <= 64 + 4 * (nnz / kWave / r->G + 1);
 }
 
 RunView view(const RunOp& o) {
@@ -1343,8 +1365,8 @@ static int build_many(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P) {
   struct Steps {
     int* p;
     ~Steps() { dev_free(p); }
-  } d_steps{(int*)dev_try_alloc(sizeof(int) * G)};
-  std::vector<int> h((size_t)G + 2);
+  } d_steps{(int*)dev_try_alloc(sizeof(int) * 2 * G)};
+  std::vector<int> h(2 * (size_t)G + 2);
   int rc = !r->r0 || !r->cs || !d_steps.p;
   bool fits = !rc;
   if (!rc) {
@@ -1355,16 +1377,18 @@ static int build_many(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P) {
                        (const int*)A->trp, (const int*)A->tci, r->r0 + G + 1);
     hipLaunchKernelGGL(k_run_cuts, dim3(grid_for((long long)(G + 1) * n, kBlock, 4096)), dim3(kBlock), 0, S(), n, G,
                        (const int*)A->trp, (const int*)A->tci, (const int*)r->r0, r->cs);
-    download(h.data(), r->r0, sizeof(int) * h.size());
+    download(h.data(), r->r0, sizeof(int) * ((size_t)G + 2));
     for (int b = 0; b < G; ++b) r->rows_max = std::max(r->rows_max, h[(size_t)b + 1] - h[(size_t)b]);
     r->lds = r->bits == 32 ? run_lds_vec<float>(n, r->rows_max, r->cw) : run_lds_vec<double>(n, r->rows_max, r->cw);
     fits = h[(size_t)G + 1] == 1 && r->rows_max < kSortMax && r->lds <= kRunLds;
   }
   if (fits) {
-    rc = build_op<kRowsA>(r, &r->A, A, d_steps.p, h.data()) || build_op<kColsA>(r, &r->At, A, d_steps.p, h.data()) ||
-         build_op<kRowsP>(r, &r->P, P, d_steps.p, h.data());
+    rc = build_op<kRowsA>(r, &r->A, A, d_steps.p, h.data());
+    if (!rc) rc = build_op<kColsA>(r, &r->At, A, d_steps.p, h.data());
+    if (!rc) rc = build_op<kRowsP>(r, &r->P, P, d_steps.p, h.data());
     for (const RunOp* o : {&r->A, &r->At, &r->P}) r->lds = ((r->lds + 15) & ~(size_t)15) + run_lds_list(o->lgT, o->ns) + 16;
-    fits = !rc && op_fits(r, r->A, A->nnz) && op_fits(r, r->At, A->nnz) && op_fits(r, r->P, P->nnz) && r->lds <= kRunLds;
+    fits = !rc && r->lds <= kRunLds;
+    if (rc == 2) rc = 0;
   }
   if (rc || !fits) {
     r->G = 0;

@@ -856,9 +856,10 @@ OSQPInt osqp_amd_solver_stats(OSQPSolver* solver, OSQPInt* pcg_iters_total, OSQP
   return 0;
 }
 
-OSQPInt osqp_amd_solver_run_stats(OSQPSolver* solver, long long* iters, OSQPInt* groups, OSQPInt* failed) {
+OSQPInt osqp_amd_solver_run_stats(OSQPSolver* solver, long long* iters, OSQPInt* groups, OSQPInt* chain,
+                                  OSQPInt* failed) {
   if (!solver || !solver->work || !solver->work->linsys_solver) return 1;
-  return osqp_amd_linsys_run_stats(solver->work->linsys_solver, iters, groups, failed);
+  return osqp_amd_linsys_run_stats(solver->work->linsys_solver, iters, groups, chain, failed);
 }
 
 OSQPInt osqp_amd_solver_run_polls(OSQPSolver* solver, OSQPInt polls) {

@@ -63,7 +63,7 @@ def load_library():
                                               C.POINTER(C.c_double)]
         lib.osqp_amd_solver_stats.restype = C.c_int
         lib.osqp_amd_solver_run_stats.argtypes = [C.POINTER(T.OSQPSolver), C.POINTER(C.c_longlong),
-                                                  C.POINTER(C.c_int), C.POINTER(C.c_int)]
+                                                  C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_int)]
         lib.osqp_amd_solver_run_stats.restype = C.c_int
         lib.osqp_amd_solver_run_polls.argtypes = [C.POINTER(T.OSQPSolver), C.c_int]
         lib.osqp_amd_solver_run_polls.restype = C.c_int
@@ -243,10 +243,11 @@ class OSQP:
 
     def run_stats(self):
         """ADMM iterations that ran many to a launch, that launch's workgroups
-        (0: the path is off) and the launches that gave up or were refused."""
-        it, g, f = C.c_longlong(), C.c_int(), C.c_int()
-        self.lib.osqp_amd_solver_run_stats(self._solver, C.byref(it), C.byref(g), C.byref(f))
-        return SimpleNamespace(iters=it.value, groups=g.value, failed=f.value)
+        (0: the path is off), the entries of a row that one lane adds up at most
+        and the launches that gave up or were refused."""
+        it, g, c, f = C.c_longlong(), C.c_int(), C.c_int(), C.c_int()
+        self.lib.osqp_amd_solver_run_stats(self._solver, C.byref(it), C.byref(g), C.byref(c), C.byref(f))
+        return SimpleNamespace(iters=it.value, groups=g.value, chain=c.value, failed=f.value)
 
     def run_polls(self, polls):
         """Looks after which such a launch's waits give up (checks)."""

@@ -177,6 +177,22 @@ def test_a_wait_that_gives_up_is_done_again(precision, check):
             assert getattr(u.info, f) == getattr(v.info, f)
 
 
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("n,m,row,long", [(400, 70000, 3, 60), (400, 70000, 3, 24), (2500, 9000, 12, 300)])
+def test_no_lane_adds_up_a_long_row(n, m, row, long, precision):
+    """Rows far longer than the average: their entries are spread over lanes, at most 24 a lane, as over the
+    lanes of a panel task, and the iterates are the separate kernels'."""
+    p = qp(n, m, row, seed=m)
+    A = p["A"].tolil()
+    for r in range(0, m, m // 40):
+        A[r, :long] = np.random.default_rng(r).standard_normal(long)
+    p["A"] = sp.csc_matrix(A)
+    a, b = both(p, precision, second=dict(q=p["q2"]), eps_abs=1e-30, eps_rel=1e-30, max_iter=40)
+    assert b[3].groups > 1 and b[3].iters == 78 and 1 <= b[3].chain <= 24
+    for u, v in zip(a[:2], b[:2]):
+        assert np.linalg.norm(u[0] - v[0]) <= (1e-9 if precision == 64 else 1e-3) * max(1.0, np.linalg.norm(u[0]))
+
+
 def test_rows_out_of_order_stay_on_the_separate_kernels(monkeypatch):
     """Columns whose rows are not ascending, as a C caller may pass them: the several-workgroup layout needs
     the order, so the solve takes the separate kernels and gives the sorted problem's answer."""
