@@ -859,6 +859,7 @@ struct HipPcg {
 
 // solves between two exact recomputations of the cached A x64
 constexpr int kZRefresh = 8;
+static_assert(kZRefresh == kRunRefresh, "a run continues this count and leaves it");
 
 template <typename V>
 const HybridOp* hyb_A(const HipPcg* s) {

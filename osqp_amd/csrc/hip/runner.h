@@ -37,6 +37,8 @@
 
 namespace osqp_hip {
 
+constexpr int kRunRefresh = 8;  // ADMM iterations between two exact recomputations of A x64
+
 struct RunOp {
   int lgT;            // log2 of the lanes per row
   int ns;             // slices per workgroup

@@ -17,7 +17,6 @@ namespace {
 constexpr int kT = 1024;            // threads of a workgroup
 constexpr int kW = kT / kWave;      // its wavefronts
 constexpr int kSortMax = 16384;     // rows of a workgroup that the layout kernel sorts
-constexpr int kRunRefresh = 8;      // ADMM iterations between two exact recomputations of A x64
 constexpr uint16_t kNoRow = 0xFFFF;
 constexpr size_t kRunLds = 159 * 1024;  // dynamic LDS of a launch
 constexpr long long kRun1Work = 48000;  // entries of A and P up to which one workgroup runs alone
@@ -686,18 +685,6 @@ __global__ __launch_bounds__(kT) void k_admm_run(RunArgs a) {
 // constraints, and the ADMM iterates part after that).  FP64 recomputes A x64
 // in every iteration, as the separate kernels do.
 
-// sum over a wavefront in the order of wave_sum's xor butterfly: the two wide
-// steps by shuffle, the rest by row rotations (lanes that a rotation swaps
-// hold equal values by then)
-__device__ __forceinline__ double wave_sum_xor(double v) {
-  v += __shfl_xor(v, 32, kWave);
-  v += __shfl_xor(v, 16, kWave);
-  v += dpp_d<0x128, 0xf>(0.0, v);  // row_ror:8, 4, 2, 1
-  v += dpp_d<0x124, 0xf>(0.0, v);
-  v += dpp_d<0x122, 0xf>(0.0, v);
-  v += dpp_d<0x121, 0xf>(0.0, v);
-  return v;
-}
 // Total of NB * 16 wavefronts' values w[]: blocks of four wavefronts added in
 // order, then the blocks by a butterfly (the partials of 256-thread blocks,
 // as the consumers of the separate kernels add them).
@@ -919,7 +906,7 @@ __global__ __launch_bounds__(kT) void k_admm_run1(RunArgs a) {
       double m1 = 0.0;
 #pragma unroll
       for (int e = 0; e < NE; ++e) {
-        const double v = wave_sum_xor((double)(yv[e] * rv[e]));
+        const double v = wave_sum((double)(yv[e] * rv[e]));
         if (lane == 0) t[e * kW + wv] = v;
         const double f = fabs((double)rv[e]);
         m1 = f > m1 ? f : m1;
@@ -970,12 +957,12 @@ __global__ __launch_bounds__(kT) void k_admm_run1(RunArgs a) {
         if (tid < n / RB)
 #pragma unroll
           for (int k = 0; k < RB; ++k) dot.add(pw[RB * tid + k] * KP[RB * tid + k]);
-        const double v = wave_sum_xor(dot.value());
+        const double v = wave_sum(dot.value());
         if (lane == 0) t[wv] = v;
       } else {
 #pragma unroll
         for (int e = 0; e < NE; ++e) {
-          const double v = wave_sum_xor((double)(pv[e] * kp[e]));
+          const double v = wave_sum((double)(pv[e] * kp[e]));
           if (lane == 0) t[e * kW + wv] = v;
         }
       }
@@ -1110,8 +1097,9 @@ const void* run_kernel_n(int n, bool res) {
   if (n <= 1 * kT) return run_kernel<V, 1>(res);
   if (n <= 2 * kT) return run_kernel<V, 2>(res);
   if (n <= 4 * kT) return run_kernel<V, 4>(res);
-  if (n <= 8 * kT || sizeof(V) == 8) return run_kernel<V, 8>(res);
-  return run_kernel<V, 12>(res);
+  if constexpr (sizeof(V) == 4)
+    if (n > 8 * kT) return run_kernel<V, 12>(res);
+  return run_kernel<V, 8>(res);  // all of FP64's
 }
 template <typename V, int NE>
 const void* run1_kernel(int res) {
