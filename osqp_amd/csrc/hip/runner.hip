@@ -19,7 +19,18 @@ constexpr int kW = kT / kWave;      // its wavefronts
 constexpr int kSortMax = 16384;     // rows of a workgroup that the layout kernel sorts
 constexpr uint16_t kNoRow = 0xFFFF;
 constexpr size_t kRunLds = 159 * 1024;  // dynamic LDS of a launch
-constexpr long long kRun1Work = 48000;  // entries of A and P up to which one workgroup runs alone
+// Entries of A and P up to which one workgroup runs alone.  us per ADMM
+// iteration (one CG iteration each) by one workgroup and by 32, FP64 / FP32:
+// 3.4k entries 20.6 / 20.1 and 29.4 / 30.0, 17k 29.9 / 26.0 and 30.2 / 29.8,
+// 26k 37.6 / 30.5 and 31.4 / 31.5, 44k 51.2 / 42.1 and 35.3 / 34.3.  The line
+// is this high for problems with equality rows, which have only the one
+// workgroup (the separate kernels take 104 and 103 at 44k); others past 20k
+// entries would be faster on 32.
+constexpr long long kRun1Work = 48000;
+// Entries up to which the runner is taken, and built (20 bytes an entry in
+// FP64, 12 in FP32): measured up to 60 M, where an iteration of 8000 x 150000
+// takes 660 us and 884 on the separate kernels (FP32 467 and 531).
+constexpr long long kRunMaxWork = 64000000;
 constexpr int kRunChain = 24;  // entries that a lane adds up of a row, while a row has lanes left to take
 constexpr int kRunPolls = 1 << 22;  // looks of a barrier's wait, some seconds
 
@@ -1401,6 +1412,7 @@ static int build_any(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P, const 
   const int n = A->n, m = A->m;
   if (A->is_triu || n <= 0 || m <= 0 || A->nnz <= 0 || n > run_n_max(bits)) return 0;
   const long long work = (long long)A->nnz + P->nnz;
+  if (work > kRunMaxWork) return 0;
   const int cus = rt().num_cu > 0 ? rt().num_cu : 256;
   int rc = 0;
   if (work <= kRun1Work && n <= 2 * kT && n + m < 65535) {
@@ -1415,7 +1427,9 @@ static int build_any(Runner* r, const OSQPMatrix* A, const OSQPMatrix* P, const 
     // Measured us per ADMM iteration with G = 32 / 64 / 128 / 256 workgroups:
     // 108k entries 33 / - / - / -, 180k 39 / 36 / 37 / 39, 624k 52 / 48 / 43 /
     // 46, 1.4M 62 / 50 / 46 / 48 (FP64): a workgroup's share against the
-    // barrier and the G shares to add.
+    // barrier and the G shares to add.  256 workgroups against the separate
+    // kernels: 5 M entries 108 and 148, 16 M 250 and 276, 30 M (8000 columns)
+    // 426 and 431, 60 M 660 and 884.
     int G = work <= 128000 ? 32 : work <= 400000 ? 64 : work <= 2000000 ? 128 : 256;
     while (G > cus) G /= 2;
     r->n = n;

@@ -111,11 +111,15 @@ int main() {
       if (allocs < least) fprintf(stderr, "FAIL %s: %d allocations\n", name, allocs), fails++;
     }
   };
-  Problem small(20, 40, 3), medium(2100, 100, 40);
+  Problem small(20, 40, 3), medium(2100, 100, 40), most(2100, 100, 40), past(2100, 100, 40);
+  most.P.nnz = 64000000 - 4000;  // the line past which it is not built
+  past.P.nnz = most.P.nnz + 1;
   for (int bits : {32, 64}) {
     tries("one workgroup", small, bits, true, bits == 32 ? 16 : 8);
     tries("several workgroups", medium, bits, false, 22);
     tries("several workgroups not asked for", medium, bits, true, 0);
+    tries("at the most entries", most, bits, false, 4);
+    tries("past the most entries", past, bits, false, 0);
   }
   printf(fails ? "FAILURES: %d\n" : "all checks passed\n", fails);
   return fails ? 1 : 0;

@@ -23,3 +23,4 @@ def test_refused_allocations_leave_the_runner_off(tmp_path):
                        env=dict(os.environ, HIP_VISIBLE_DEVICES="-1", ROCR_VISIBLE_DEVICES="-1"))
     assert r.returncode == 0 and "all checks passed" in r.stdout, r.stdout[-2000:] + r.stderr[-2000:]
     assert "not asked for, 64 bits, one 1: 0 allocations" in r.stdout
+    assert "past the most entries, 64 bits, one 0: 0 allocations" in r.stdout
