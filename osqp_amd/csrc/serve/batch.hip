@@ -356,9 +356,9 @@ constexpr int kSlicedBucket = 3;
 // Problems of the buckets below kLaneBuckets whose rows of P and A' have at
 // most kLaneRow entries, and those of A too or more than kLongRow, run in
 // buckets of their own (kBuckets + size bucket), on the kernel over lane rows:
-// 512 MPC problems of horizons 10..50 from 60.0 to 31.9 ms (FP32), 24 of them
-// from 18.6 to 10.7 ms (FP64), 12 resident portfolios of 500..1000 assets from
-// 621 to 300 ms, the same bits.  A row in between has more pieces than the
+// 512 MPC problems of horizons 10..50 from 56.5 to 32.9 ms (FP32), 24 of them
+// from 18.3 to 10.5 ms (FP64), 12 resident portfolios of 500..1000 assets from
+// 662 to 341 ms, the same bits (with lane_admm and the register reductions).  A row in between has more pieces than the
 // left-to-right sum keeps in the group walk's order.  Up to kLaneCols columns
 // the ADMM step laid out for lane rows takes them (Solver::lane_admm, FP64: one
 // reduction block a wavefront); past that only FP32, and only rows that the
@@ -368,7 +368,9 @@ constexpr int kSlicedBucket = 3;
 // 1.17, FP64 1.27 / 1.38 / 1.20, 1.10 / 1.16 / 1.02, 1.37 / 1.40 / 1.11;
 // n = 3000 FP32 1.17 / 1.15 / 0.96, 1.30 / 1.31 / 1.05, 1.58 / 1.58 / 1.22,
 // FP64 0.63 / 0.88 / 0.74, 0.93 / 0.85 / 0.90, 0.91 / 0.97 / 0.97.  Slots over
-// entries there: 5.4, 3.2, 2.0.
+// entries there: 5.4, 3.2, 2.0.  (Where the GPU is full the padding counts most:
+// 512 to 2048 problems of 1000 columns and rows of 3 entries take 0.91 of the row
+// groups' speed in FP64 and 1.0 in FP32, of 500 and 2000 columns 0.99 to 1.06.)
 constexpr int kLaneBuckets = 3;
 constexpr int kLaneCols = kMaxTeamWaves * kRedBlock;
 constexpr double kLanePad = 4.5;
@@ -918,6 +920,10 @@ constexpr int kSmallBuckets = 2;
 // The lane buckets try the candidates of 256 and 512 threads: one horizon-50
 // problem's iteration takes 78 us with 256 threads and 58 with 512, a horizon-10
 // one's 34 and 32; a 1000-asset portfolio's 215 and 166, with 64 threads 657.
+// Bulks of tiny problems keep their throughput on them: a list of 16384 QPs of
+// 4, 16 and 48 columns took 318, 424 and 471 ms in FP32 on row groups, whose
+// tuner chose 64 and 128 threads, and 321, 384 and 398 on lane rows (FP64 337,
+// 427, 471 and 328, 419, 440); 512 of 64 columns 60 and 34 ms.
 constexpr int kLaneCand0 = 2;
 inline int cands_of(int bucket) {
   return bucket >= kBuckets ? kNumCands - kLaneCand0 : bucket < kSmallBuckets ? 4 : kNumCands;
