@@ -3,7 +3,8 @@
 // visible).  Device memory is host memory here and no kernel runs: for every
 // allocation of the two builds, the build is tried with that allocation
 // refused, and with an exception in its place; each time the runner must come
-// back off and empty, with every block given back and nothing recorded.
+// back off and empty, with every block given back and nothing recorded.  A
+// launch that is refused (without a GPU all are) must be reported by runner_run.
 #include "hip/runner.hip"
 
 #include <set>
@@ -120,6 +121,21 @@ int main() {
     tries("several workgroups not asked for", medium, bits, true, 0);
     tries("at the most entries", most, bits, false, 4);
     tries("past the most entries", past, bits, false, 0);
+  }
+  for (int groups : {1, 32}) {
+    Runner r;
+    memset(&r, 0, sizeof(r));
+    r.on = 1;
+    r.n = 20;
+    r.m = 40;
+    r.bits = 64;
+    r.G = groups;
+    RunCall c;
+    memset(&c, 0, sizeof(c));
+    c.iters = 24;
+    int z = -7;
+    if (!runner_run(&r, &small.A, &small.P, small.K, c, &z) || z != -7)
+      fprintf(stderr, "FAIL: a refused launch of %d workgroups went unnoticed\n", groups), fails++;
   }
   printf(fails ? "FAILURES: %d\n" : "all checks passed\n", fails);
   return fails ? 1 : 0;
