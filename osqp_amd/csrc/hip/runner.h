@@ -23,6 +23,8 @@
 //     L2s, and the matrix stays cached.  Measured on 256 workgroups: 2.6 us a
 //     barrier, 17.9 us with fences.
 //   * With G = 1 the barriers are workgroup barriers.
+//   * A barrier's wait is bounded; what a launch changes is copied before it
+//     (3 us), so that a launch that gave up can be done again elsewhere.
 //
 // P's rows of a chunk belong to the chunk's workgroup.  The copies are sliced: 64 lanes hold 64 / T rows, T lanes a row, rows
 // of a workgroup sorted by length (longest first) so that a slice's width is
@@ -37,7 +39,12 @@
 
 namespace osqp_hip {
 
-constexpr int kRunRefresh = 8;  // ADMM iterations between two exact recomputations of A x64
+// ADMM iterations between two exact recomputations of A x64 (one workgroup in
+// FP64: every one).  Against 80-bit arithmetic the vector carried in between has
+// 1.08 to 1.45 times a fresh product's relative error of 1.3e-16 to 3.5e-16
+// (n = 300..5000); a product in every iteration took 5000 x 50000 in FP64 from
+// 172 to 189 ms, with outputs that differ by 1e-15.
+constexpr int kRunRefresh = 8;
 
 struct RunOp {
   int lgT;            // log2 of the lanes per row
